@@ -902,6 +902,11 @@ int nbx_set_nonbonded_parameters(nbx_context* c, int numTypes, const double* c6,
         }
         c->typeLJ.ensure(t);
         check(hipMemcpy(c->typeLJ.p, lj.data(), sizeof(int) * t, hipMemcpyHostToDevice), "upload LJ flags");
+        c->ljMask = 0;
+        for (int i = 0; i < t; i++)
+        {
+            c->ljMask |= lj[i] ? 1ull << i : 0ull;
+        }
         c->anyTypeWithoutLJ = std::count(lj.begin(), lj.end() - 1, 0) > 0;
         c->c6diag.assign(t, 0.0f);
         for (int i = 0; i < t; i++)
@@ -1506,7 +1511,7 @@ static void enqueueStep(nbx_context* c, unsigned flags, const float* xd, float* 
     a.xq            = c->xq.p;
     a.type          = c->nbtype.p;
     a.nbfp          = c->nbfp.p;
-    a.typeLJ        = c->typeLJ.p;
+    a.ljMask        = c->ljMask;
     a.skipLJ        = c->anyTypeWithoutLJ ? 1 : 0;
     a.vdwModifier   = c->opt.vdw_modifier;
     a.ljPme         = c->opt.vdw_type == NBX_VDW_PME ? 1 : 0;

@@ -308,6 +308,7 @@ struct nbx_context
     // the first adjoint call after a search)
     nbx::DevBuf<int>    statsPartial; // per-workgroup maxima (launchPartialMax)
     nbx::DevBuf<int>    typeLJ; // per type (padding type included): 1 if it has LJ with any type
+    unsigned long long  ljMask = 0; // typeLJ as bits (at most kMaxTypes + 1 types)
     bool                anyTypeWithoutLJ = false; // among the user's types
     // LJ-PME: the grid's 6 C6 per type pair; the host's 6 C6 diagonal and
     // the per-type atom counts give the self energy

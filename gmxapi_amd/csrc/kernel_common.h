@@ -56,6 +56,18 @@ __device__ __forceinline__ int uniformInt(int v)
     return __builtin_amdgcn_readfirstlane(v);
 }
 
+// Wave-uniform reads through the scalar unit: 64- or 16-byte records at a
+// wave-uniform address of memory that the launch does not write.
+using Float16 = float __attribute__((ext_vector_type(16)));
+using Int4    = int __attribute__((ext_vector_type(4)));
+
+template<typename V, typename T>
+__device__ __forceinline__ V scalarLoad(const T* p)
+{
+    using Constant = const __attribute__((address_space(4))) V;
+    return *(Constant*)(p);
+}
+
 // The four i-atoms of the current i-entry, wave-uniform (scalar registers):
 // coordinates and charge as stored, and LJ table row offsets.
 struct IAtoms

@@ -91,8 +91,10 @@ __host__ __device__ inline int adjointLayoutBudget(int ntype)
 {
     return kAdjointLayoutBudget + (adjointAccCopies(ntype) - 1) * ntype * ntype * 16;
 }
-// rsq floor for float (pairlist.h:146): r > 6.2e-4 nm
+// rsq floor for float (pairlist.h:146): r > 6.2e-4 nm; and a cap far beyond
+// any cut-off that keeps products of the masked 1/r = 0 finite
 constexpr float kMinRsq = 3.82e-07f;
+constexpr float kMaxRsq = 1e30f;
 
 // Coulomb flavours of the kernel
 enum Elec : int
@@ -428,7 +430,7 @@ struct KernelArgs
     const float4* xq;
     const int*    type;
     const float2* nbfp;
-    const int*    typeLJ; // per type: 1 if it has LJ with any type
+    unsigned long long ljMask; // bit t: type t has LJ with any type
     int           skipLJ; // host: some type has no LJ (launch the variant that skips it)
     int           vdwModifier; // host: NBX_VDW_* modifier
     int           ljPme;       // host: LJ-PME (c6grid is read)
@@ -468,6 +470,13 @@ hipError_t allowDynamicLds(const void* fn, int lds);
 // start/stop (either may be NULL) record the launch's own start and end
 hipError_t launchNonbonded(hipStream_t s, const KernelArgs& a, int elec, bool energy, bool shiftForces, int numBlocks,
                            hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
+// one Coulomb flavour's instantiations, with the LJ flavour chosen from a
+hipError_t launchNonbondedRF(hipStream_t s, const KernelArgs& a, bool energy, bool shiftForces, int numBlocks, int lds,
+                             hipEvent_t start, hipEvent_t stop);
+hipError_t launchNonbondedTable(hipStream_t s, const KernelArgs& a, bool energy, bool shiftForces, int numBlocks,
+                                int lds, hipEvent_t start, hipEvent_t stop);
+hipError_t launchNonbondedAnalytical(hipStream_t s, const KernelArgs& a, bool energy, bool shiftForces, int numBlocks,
+                                     int lds, hipEvent_t start, hipEvent_t stop);
 int  nonbondedLdsBytes(int ntype, int tabN, int elec, int windowSlots, bool ljPme = false);
 
 // -- adjoint.hip

@@ -1,0 +1,55 @@
+"""The forces-only pair kernel against the energy kernel and the oracle at
+sizes where its tiles, windows and table reads have edges."""
+import numpy as np
+import pytest
+
+from gmxapi_amd import nbx, systems as S
+from tests.helpers import oracle_for, rms
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(name):
+    if name == "water70":  # fewer clusters than wavefronts, one-tile i-entries
+        return S.water_box(70, 2.05, seed=3, rc=0.9, rlist=1.0)
+    if name == "water1001":
+        return S.water_box(1001, None, seed=4)
+    return S.hetero_chains(2410, 2.9, ntypes=7, seed=5)  # rc 1.2: windows overflow
+
+
+@pytest.mark.parametrize("options", [dict(), dict(ewald_correction="analytical"), dict(coulomb="reaction-field"),
+                                     dict(vdw_modifier="force-switch", rvdw_switch=0.7)],
+                         ids=["table", "analytical", "rf", "force-switch"])
+@pytest.mark.parametrize("name", ["water70", "water1001", "chains2410"])
+def test_forces_only_kernel_matches_energy_kernel(name, options):
+    # the two kernels round the same pair terms in another order and, with
+    # the table, read it at positions that differ by the rounding of
+    # r * scale + 1 (6e-5 of an entry, 1.3e-6 of the correction's force):
+    # a few 1e-7 of the RMS force, here bounded by 4e-6
+    print(f"[forces only] {name} {options}", flush=True)
+    s = _system(name)
+    ctx = nbx.context_for(s, **options)
+    f = ctx.compute(s.x)
+    fe = ctx.compute(s.x, energy=True)
+    assert rms(f - fe) <= 4e-6 * rms(fe)
+    if not options:
+        r64 = oracle_for(s, "f64").compute(s.x)
+        assert rms(f - r64["f"]) <= 5e-4 * rms(r64["f"])
+
+
+@pytest.mark.parametrize("far", [1e6, 1e19, 3e38])
+def test_atom_far_outside_leaves_the_others_finite(far):
+    # an atom that has left the box by any float distance is beyond every
+    # cut-off: the atoms listed with it keep the forces they have without it
+    print(f"[far atom] {far}", flush=True)
+    s = S.water_box(500, None, seed=6)
+    ctx = nbx.context_for(s)
+    x = s.x.astype(np.float32)
+    x[7] = (1e5, 1e5, 1e5)
+    near = ctx.compute(x)
+    x[7] = (far, far, -far)
+    others = np.arange(s.natoms) != 7
+    for energy in (False, True):
+        f = ctx.compute(x, energy=energy)
+        assert np.isfinite(f[others]).all()
+        assert rms(f[others] - near[others]) <= 4e-6 * rms(near[others])
