@@ -311,6 +311,38 @@ static void ensureStats(nbx_context* c)
     c->statsPartial.ensure(kStatsHead + kPartialMaxBlocks * partialMaxStride(2, true));
 }
 
+// The group size beyond which larger groups stage more.  Every (wavefront,
+// group) pair clears, stages and gathers one window, and every wavefront but
+// the first starts inside some group, so (nc / G + waves) windows of U(G) + G
+// slots are moved.  U(G), the distinct j-clusters of G consecutive clusters,
+// is close to (0.87 + 0.15 G) times the j-entries per cluster (288,000-atom
+// water: 95, 150, 216, 333 slots for G = 1, 4, 8, 16; 150,000-atom chains: 166,
+// 239, 325, 472).  Large systems take the largest G that fits; where the
+// wavefronts outnumber the groups a small one: 9,000 waters' atoms G = 2
+// instead of 16, half the staged bytes.
+int stagedGroupSize(const nbx_context* c, bool adjoint)
+{
+    const double nc = std::max(c->ncluster, 1);
+    const double nj = static_cast<double>(c->ncj) / nc;
+    // the wavefronts of the launch: two per SIMD for the pair kernel (three
+    // two-wavefront workgroups per CU for the adjoint), or this system's
+    // share of a batch's launch
+    const double resident = c->numCU * (adjoint ? 6.0 : 2.0 * kKernelWaves);
+    const double waves    = !adjoint && c->batchWaves > 0 ? c->batchWaves : std::min(resident, std::max(1.0, 1.0 * c->nci));
+    double       least    = 0.0;
+    int          best     = 1;
+    for (int G = 1; G <= kGroupSizeMax; G *= 2)
+    {
+        const double staged = (nc / G + waves) * (nj * (0.87 + 0.15 * G) + G);
+        if (G == 1 || staged < least)
+        {
+            least = staged;
+            best  = G;
+        }
+    }
+    return best;
+}
+
 // Groups of consecutive i-clusters for the kernel's LDS j-force window
 // (groups.hip): the largest group size whose j-entries fit the LDS sort and
 // whose window fits the kernel's LDS budget (the pair kernel's, or with
@@ -340,9 +372,10 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
         reducePartialMax(hp, nb, kGroupSizeCount, spans);
     }
     c->jentryTmp.ensure(c->ncj);
-    // the largest group size (or the chosen one) whose j-force windows, one
-    // per wavefront, fit the workgroup's LDS budget: larger groups share more
-    // j-clusters per flush, which pays more than a third resident workgroup.
+    // the largest group size up to stagedGroupSize (or the chosen one) whose
+    // j-force windows, one per wavefront, fit the workgroup's LDS budget:
+    // larger groups share more j-clusters per flush, which pays more than a
+    // third resident workgroup.
     // When no size fits with at most 2% of the union entries spilled to
     // global atomics (long cut-offs, many types), the last pass takes the
     // smallest (or the chosen) size with whatever spill its window leaves.
@@ -354,8 +387,9 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
     // a layout rebuilt for a new list starts from the size its last build
     // chose: the sizes above it did not fit then and, for a system that
     // moved by a few steps, do not fit now (saves a count pass per search)
-    int first = 0;
-    while (forced <= 0 && L.groupSize > 0 && first < kGroupSizeCount - 1 && (kGroupSizeMax >> first) > L.groupSize)
+    const int largest = L.groupSize > 0 ? std::min(L.groupSize, stagedGroupSize(c, adjoint)) : stagedGroupSize(c, adjoint);
+    int       first   = 0;
+    while (forced <= 0 && first < kGroupSizeCount - 1 && (kGroupSizeMax >> first) > largest)
     {
         first++;
     }
@@ -1017,7 +1051,8 @@ int nbx_set_topology(nbx_context* c, int numAtoms, const int* types, const float
             }
         }
         setDevice(c);
-        c->natoms = numAtoms;
+        c->natoms        = numAtoms;
+        c->lay.groupSize = c->adj.groupSize = 0; // another system: its layouts choose anew
         c->type.ensure(numAtoms);
         c->charge.ensure(numAtoms);
         c->exclOff.ensure(numAtoms + 1);

@@ -145,9 +145,16 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
     {
         throw StateError("the batch holds no systems");
     }
+    // the launch's wavefronts (two workgroups per CU) by the members' sizes
+    long long batchClusters = 1;
+    for (nbx_context* c : b->sys)
+    {
+        batchClusters += c->ncluster;
+    }
     for (nbx_context* c : b->sys)
     {
         c->opt.kernel_group_size = G;
+        c->batchWaves = 1 + static_cast<int>(2LL * kKernelWaves * b->numCU * c->ncluster / batchClusters);
         statusCheck(nbx_construct_pairlist(c), "nbx_construct_pairlist");
     }
     check(hipSetDevice(b->device), "hipSetDevice");

@@ -252,6 +252,7 @@ struct nbx_context
     std::vector<hipEvent_t> timingEvents; // start, stop pairs
     int                     timingRecorded = 0;
     int              numCU      = 256;
+    int              batchWaves = 0; // a batch member: its share of the launch's wavefronts
     int              elec       = nbx::kElecEwaldTable;
     nbx::InteractionConst ic{};
     double           selfCoef = 0.0;

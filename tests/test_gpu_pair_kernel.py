@@ -53,3 +53,20 @@ def test_atom_far_outside_leaves_the_others_finite(far):
         f = ctx.compute(x, energy=energy)
         assert np.isfinite(f[others]).all()
         assert rms(f[others] - near[others]) <= 4e-6 * rms(near[others])
+
+
+@pytest.mark.parametrize("molecules", [280, 1000, 3000, 9001])
+def test_group_size_rule_keeps_forces(molecules):
+    # the group size chosen for the system's size (1, 2, 4, ... as the
+    # clusters outgrow the wavefronts) against a forced one: the same pair
+    # terms, summed in another order (float sums of a few hundred terms)
+    s = S.water_box(molecules, None, seed=molecules)
+    ctx = nbx.context_for(s)
+    print(f"[group size] {molecules} molecules: {ctx.work_groups()['group_size']}", flush=True)
+    f = ctx.compute(s.x, energy=True)
+    e = ctx.energies()
+    for forced in (1, 8):
+        other = nbx.context_for(s, kernel_group_size=forced)
+        g = other.compute(s.x, energy=True)
+        assert rms(f - g) <= 4e-6 * rms(g)
+        np.testing.assert_allclose(e, other.energies(), rtol=1e-6)
