@@ -410,20 +410,39 @@ __global__ __launch_bounds__(kGatherThreads) void gatherForcesKernel(int ncluste
     const int lb = gridDim.x % kGatherXcds == 0
                        ? (blockIdx.x % kGatherXcds) * (gridDim.x / kGatherXcds) + blockIdx.x / kGatherXcds
                        : blockIdx.x;
-    for (int c = lb * kWaves + wave; c < ncluster; c += gridDim.x * kWaves)
+    // A cluster's copies are three dependent reads away (its range in gpos,
+    // the positions, the copies), and a wavefront takes several clusters in
+    // turn: the positions of the next cluster and the range of the one after
+    // it are read while a cluster's copies are summed.
+    const int stride = gridDim.x * kWaves;
+    const int first  = lb * kWaves + wave;
+    auto      range  = [&](int c) {
+        return c < ncluster ? make_int2(gposOff[c], gposOff[c + 1]) : make_int2(0, 0);
+    };
+    auto position = [&](int2 r) { return r.x + lane < r.y ? gpos[r.x + lane] : -1; };
+    int2 cur  = range(first);
+    int2 next = range(first + stride);
+    int  pCur = position(cur);
+    for (int c = first; c < ncluster; c += stride)
     {
-        float f[12];
+        const int2 after = range(c + 2 * stride);
+        const int  pNext = position(next);
+        // this lane's component of the sum (lanes past the 12th repeat it)
+        const int slot = c * kClusterSize + min(idx, 11) / 3;
+        const int a    = kToAtoms ? atomIndices[slot] : 0;
+        float     f[12];
 #pragma unroll
         for (int k = 0; k < 12; k++)
         {
             f[k] = 0.0f;
         }
-        for (int i = gposOff[c] + lane; i < gposOff[c + 1]; i += 64)
+        int p = pCur;
+        for (int i = cur.x + lane; i < cur.y; i += 64)
         {
-            const int    p  = gpos[i];
             const float4 v0 = staging[p];
             const float4 v1 = staging[p + 1];
             const float4 v2 = staging[p + 2];
+            p               = i + 64 < cur.y ? gpos[i + 64] : 0;
             f[0] += v0.x;
             f[1] += v0.y;
             f[2] += v0.z;
@@ -437,18 +456,19 @@ __global__ __launch_bounds__(kGatherThreads) void gatherForcesKernel(int ncluste
             f[10] += v2.z;
             f[11] += v2.w;
         }
+        cur  = next;
+        next = after;
+        pCur = pNext;
         // lane L ends up with component L >> 2 = 3 * atom + d
         const float r = waveReduceScatter12(f, lane);
         if ((lane & 3) == 0 && idx < 12)
         {
-            const int slot = c * kClusterSize + idx / 3;
-            float*    dst  = fnb ? reinterpret_cast<float*>(fnb + slot) + idx % 3 : nullptr;
+            float* dst = fnb ? reinterpret_cast<float*>(fnb + slot) + idx % 3 : nullptr;
             // the fixed-point sums of the window overflow, if any
             const float over = fixF ? fromFixed(fixF[3 * slot + idx % 3]) : 0.0f;
             if (kToAtoms)
             {
                 // straight to the caller's atom-order forces (nbat-f -> f)
-                const int a = atomIndices[slot];
                 if (a >= 0)
                 {
                     const float fv = (fnb ? *dst : 0.0f) + (r + over);
@@ -456,10 +476,10 @@ __global__ __launch_bounds__(kGatherThreads) void gatherForcesKernel(int ncluste
                     *fo            = addToF ? *fo + fv : fv;
                     if (virPart)
                     {
-                        const float4 p = xq[slot];
-                        vir[0] += static_cast<double>(p.x) * fv;
-                        vir[1] += static_cast<double>(p.y) * fv;
-                        vir[2] += static_cast<double>(p.z) * fv;
+                        const float4 q = xq[slot];
+                        vir[0] += static_cast<double>(q.x) * fv;
+                        vir[1] += static_cast<double>(q.y) * fv;
+                        vir[2] += static_cast<double>(q.z) * fv;
                     }
                 }
             }
