@@ -1229,10 +1229,8 @@ static void finishList(nbx_context* c, const int* spans = nullptr)
     c->energyPartial.ensure(2 * static_cast<size_t>(c->lay.ngroups + numWaves));
     c->exclPartial.ensure(kExclMaxBlocks);
     c->fshiftPartial.ensure(static_cast<size_t>(c->lay.numBlocks) * kNumShifts * 3);
-    c->energy.ensure(2);
-    c->fshift.ensure(kNumShifts * 3);
+    c->results.ensure(kResults);
     c->virialPartial.ensure(9 * static_cast<size_t>(kGatherMaxBlocks));
-    c->virial.ensure(9);
     c->listValid  = true;
     c->adjValid   = false;
     c->layOuterValid = false;
@@ -1606,13 +1604,27 @@ static void enqueueStep(nbx_context* c, unsigned flags, const float* xd, float* 
     if (energy || shift || virial)
     {
         launchFinalize(c->stream, energy ? numSlots : 0, c->energyPartial.p, energy ? numExcl : 0,
-                       c->exclPartial.p, c->lay.numBlocks, c->fshiftPartial.p, shift, c->energy.p, c->fshift.p,
-                       virial ? numVir : 0, c->virialPartial.p, c->shiftVec.p, virial ? c->virial.p : nullptr);
+                       c->exclPartial.p, c->lay.numBlocks, c->fshiftPartial.p, shift, c->results.p, c->results.p + kResultShift,
+                       virial ? numVir : 0, c->virialPartial.p, c->shiftVec.p, virial ? c->results.p + kResultVirial : nullptr);
     }
     check(hipGetLastError(), "nonbonded kernel");
     c->haveEnergy = energy;
     c->haveShift  = shift;
     c->haveVirial = virial;
+    c->resultsRead = false;
+}
+
+// The step's results in host memory: one wait for the first getter after a
+// step, none for the others.
+static const double* stepResults(nbx_context* c)
+{
+    if (!c->resultsRead)
+    {
+        setDevice(c);
+        check(hipStreamSynchronize(c->stream), "sync");
+        c->resultsRead = true;
+    }
+    return c->results.p;
 }
 
 int nbx_dispatch_kernel(nbx_context* c, unsigned flags)
@@ -1857,14 +1869,10 @@ int nbx_get_energies(nbx_context* c, double* vlj, double* vc)
         {
             throw StateError("no energies: compute with NBX_COMPUTE_ENERGY first");
         }
-        setDevice(c);
-        double e[2];
-        check(hipMemcpyAsync(e, c->energy.p, sizeof(e), hipMemcpyDeviceToHost, c->stream), "read energies");
-        check(hipStreamSynchronize(c->stream), "sync");
-        e[0] += ljPmeSelfEnergy(c);
+        const double* e = stepResults(c);
         if (vlj)
         {
-            *vlj = e[0];
+            *vlj = e[0] + ljPmeSelfEnergy(c);
         }
         if (vc)
         {
@@ -1884,10 +1892,12 @@ int nbx_get_shift_forces(nbx_context* c, double* fshift)
         {
             throw StateError("no shift forces: compute with NBX_COMPUTE_SHIFT_FORCES first");
         }
-        setDevice(c);
-        check(hipMemcpyAsync(fshift, c->fshift.p, sizeof(double) * kNumShifts * 3, hipMemcpyDeviceToHost, c->stream),
-              "read fshift");
-        check(hipStreamSynchronize(c->stream), "sync");
+        if (!fshift)
+        {
+            throw DeviceError("read fshift: the output must not be NULL");
+        }
+        const double* r = stepResults(c);
+        std::copy(r + kResultShift, r + kResultVirial, fshift);
     });
 }
 
@@ -1902,9 +1912,12 @@ int nbx_get_virial(nbx_context* c, double* virial)
         {
             throw StateError("no virial: compute with NBX_COMPUTE_VIRIAL first");
         }
-        setDevice(c);
-        check(hipMemcpyAsync(virial, c->virial.p, sizeof(double) * 9, hipMemcpyDeviceToHost, c->stream), "read virial");
-        check(hipStreamSynchronize(c->stream), "sync");
+        if (!virial)
+        {
+            throw DeviceError("read virial: the output must not be NULL");
+        }
+        const double* r = stepResults(c);
+        std::copy(r + kResultVirial, r + kResults, virial);
     });
 }
 

@@ -47,7 +47,8 @@ struct nbx_batch
     WindowGather   gather;
     DevBuf<uint2>  work;
     DevBuf<int4>   chunks, groups, groupInfo;
-    DevBuf<double> energyPartial, atomEnergy, energy;
+    DevBuf<double> energyPartial, atomEnergy;
+    PinnedBuf<double> energy; // per system {LJ, Coulomb}, written by the step's final sums
     bool           haveEnergy = false;
 
     hipGraph_t     graph     = nullptr;
@@ -575,8 +576,7 @@ int nbx_batch_get_energies(nbx_batch* b, double* energies)
         }
         check(hipSetDevice(b->device), "hipSetDevice");
         check(hipStreamSynchronize(b->stream), "sync");
-        check(hipMemcpy(energies, b->energy.p, 2 * b->sys.size() * sizeof(double), hipMemcpyDeviceToHost),
-              "read energies");
+        std::copy(b->energy.p, b->energy.p + 2 * b->sys.size(), energies);
         for (size_t r = 0; r < b->sys.size(); r++)
         {
             energies[2 * r] += ljPmeSelfEnergy(b->sys[r]);

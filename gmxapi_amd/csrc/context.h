@@ -99,6 +99,42 @@ struct DevBuf
     ~DevBuf() { release(); }
 };
 
+// Pinned host memory that kernels write directly: a step's few results need no
+// copy behind the kernels, only the wait for the stream.
+template<typename T>
+struct PinnedBuf
+{
+    T*     p   = nullptr;
+    size_t cap = 0;
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf&) = delete;
+    PinnedBuf& operator=(const PinnedBuf&) = delete;
+    void ensure(size_t n)
+    {
+        if (n <= cap && p)
+        {
+            return;
+        }
+        if (p)
+        {
+            check(hipHostFree(p), "hipHostFree");
+            p   = nullptr;
+            cap = 0;
+        }
+        void* q = nullptr;
+        check(hipHostMalloc(&q, std::max<size_t>(n, 1) * sizeof(T), hipHostMallocDefault), "hipHostMalloc");
+        p   = static_cast<T*>(q);
+        cap = std::max<size_t>(n, 1);
+    }
+    ~PinnedBuf()
+    {
+        if (p)
+        {
+            (void)hipHostFree(p);
+        }
+    }
+};
+
 // The pair kernel's staged j-force windows and the lists that gather them
 // (one per context, one per batch).
 struct WindowGather
@@ -329,7 +365,11 @@ struct nbx_context
     bool                adjValid = false;
 
     // outputs
-    nbx::DevBuf<double>  energyPartial, energy, fshift, virialPartial, virial;
+    nbx::DevBuf<double>  energyPartial, virialPartial;
+    // the last step's results, written by its final sums: energies,
+    // shift forces, virial
+    nbx::PinnedBuf<double> results;
+    bool                   resultsRead = false; // the stream was waited for since that step
     nbx::DevBuf<double>  exclPartial;
     nbx::DevBuf<float>   fshiftPartial, fOut;
     // adjoint
@@ -338,6 +378,13 @@ struct nbx_context
     nbx::DevBuf<float>   gIn, gradXOut;
     bool            haveEnergy = false, haveShift = false, haveVirial = false;
 };
+
+namespace nbx
+{
+constexpr int kResultShift  = 2;                             // after the two energies
+constexpr int kResultVirial = kResultShift + 3 * kNumShifts; // after the shift forces
+constexpr int kResults      = kResultVirial + 9;
+} // namespace nbx
 
 // LJ-PME self energy, 0.5 C6_ii beta_lj^6 / 6 per atom
 // (kernel_ref_outer.h:315-322): a constant of the topology and parameters,

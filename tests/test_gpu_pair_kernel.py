@@ -70,3 +70,31 @@ def test_group_size_rule_keeps_forces(molecules):
         g = other.compute(s.x, energy=True)
         assert rms(f - g) <= 4e-6 * rms(g)
         np.testing.assert_allclose(e, other.energies(), rtol=1e-6)
+
+
+def test_results_follow_the_last_step():
+    # energies, virial and shift forces are those of the last step, whichever
+    # is read first and however many steps ran since the last read
+    s = S.water_box(1001, None, seed=4)
+    moved = (s.x + 0.01 * np.random.default_rng(1).normal(size=s.x.shape)).astype(np.float32)
+
+    def results(ctx, order):
+        read = dict(e=lambda: np.array(ctx.energies()), v=ctx.virial, f=ctx.shift_forces)
+        got = {k: read[k]() for k in order}
+        return [got[k] for k in "evf"]
+
+    flags = dict(energy=True, virial=True, shift_forces=True, reproducible=True)
+    want = []
+    for x in (s.x, moved):
+        ctx = nbx.context_for(s)
+        ctx.compute(x, **flags)
+        want.append(results(ctx, "evf"))
+    ctx = nbx.context_for(s)
+    for which, order in ((0, "vef"), (1, "fve"), (0, "efv")):
+        ctx.compute((s.x, moved)[1 - which], **flags)
+        ctx.compute((s.x, moved)[which], **flags)
+        for a, b in zip(results(ctx, order), want[which]):
+            np.testing.assert_array_equal(a, b)
+    ctx.compute(s.x)
+    with pytest.raises(nbx.NbxStateError):
+        ctx.energies()
