@@ -15,6 +15,7 @@
 // A step (coordinate conversion, force clearing, pair kernel, exclusion
 // energies, per-system sums, force reduction) is launch-bound for small
 // systems and can be recorded once into a HIP graph and replayed.
+#include <climits>
 #include <cstring>
 #include <numeric>
 
@@ -43,6 +44,7 @@ struct nbx_batch
     DevBuf<unsigned long long> fixF; // window-overflow forces in fixed point, 3 per atom slot
     DevBuf<int>    nbtype, atomIndices, cells, exclOff, exclIdx, unionList, atomSystem, groupOff, atomOff, slotOff;
     DevBuf<int2>   waveStart;
+    DevBuf<int>    chunkCost, costOff; // the schedule's per-chunk costs (and their total) and their scan
     DevBuf<float>  boxes;
     WindowGather   gather;
     DevBuf<uint2>  work;
@@ -127,8 +129,25 @@ void scheduleBatch(nbx_batch* b, int blocksPerCU, int chunkWeight)
     b->waveStart.ensure(numWaves + 1);
     b->slotOff.ensure(R + 1);
     b->energyPartial.ensure(2 * static_cast<size_t>(b->ngroups + numWaves));
-    launchWaveSchedule(b->stream, numWaves, b->nchunk, b->chunks.p, b->nwork, chunkWeight, b->ngroups, b->groups.p,
-                       b->waveStart.p, nullptr, nullptr, b->numCU * kKernelWaves);
+    // the single system's cost model (LJ i-atoms counted), with chunkWeight
+    // work entries per chunk; by work entries alone if the total could
+    // overflow an int
+    const int chunkCost = chunkWeight * kCostTile / kTileJ;
+    if (scheduleCostBound(b->nwork, b->nchunk, chunkCost) < INT_MAX)
+    {
+        b->chunkCost.ensure(b->nchunk + 2);
+        b->costOff.ensure(scanOutSize(b->nchunk));
+        launchChunkCosts(b->stream, b->nchunk, b->chunks.p, b->nbtype.p, c0->typeLJ.p, chunkCost, b->chunkCost.p);
+        launchExclusiveScanWide(b->stream, b->nchunk, b->chunkCost.p, b->costOff.p, b->chunkCost.p + b->nchunk + 1);
+        launchWaveSchedule(b->stream, numWaves, b->nchunk, b->chunks.p, b->nwork, chunkWeight, b->ngroups,
+                           b->groups.p, b->waveStart.p, b->costOff.p, b->chunkCost.p + b->nchunk + 1,
+                           b->numCU * kKernelWaves);
+    }
+    else
+    {
+        launchWaveSchedule(b->stream, numWaves, b->nchunk, b->chunks.p, b->nwork, chunkWeight, b->ngroups,
+                           b->groups.p, b->waveStart.p, nullptr, nullptr, b->numCU * kKernelWaves);
+    }
     launchSystemSlots(b->stream, R, b->groupOff.p, b->ngroups, b->groups.p, numWaves, b->waveStart.p, b->slotOff.p);
     check(hipGetLastError(), "schedule kernels");
     buildSegments(b->stream, b->gather, b->ngroups, b->groups.p, b->groupInfo.p, numWaves, b->waveStart.p,
@@ -611,7 +630,7 @@ int nbx_batch_autotune(nbx_batch* b, const float* x, float* f, unsigned flags, i
             const int fitBpc = b->blocksPerCU;
             for (int bpc = fitBpc; bpc >= 2; bpc--)
             {
-                for (int weight : { kChunkWeight, 4 * kChunkWeight })
+                for (int weight : { kChunkWeight, 2 * kChunkWeight })
                 {
                     scheduleBatch(b, bpc, weight);
                     enqueueCompute(b, x, f, flags); // warm-up

@@ -882,7 +882,7 @@ __global__ void chunkShiftKernel(int nchunk, const int4* __restrict__ chunks, co
 // reduction).  Fitted to the run times of individual wavefronts on the
 // 288,000-atom water box, where it leaves 2.3 us of 205 us unexplained.
 __global__ void chunkCostKernel(int nchunk, const int4* __restrict__ chunks, const int* __restrict__ type,
-                                const int* __restrict__ typeLJ, int* __restrict__ cost)
+                                const int* __restrict__ typeLJ, int chunkCost, int* __restrict__ cost)
 {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m < nchunk)
@@ -894,16 +894,19 @@ __global__ void chunkCostKernel(int nchunk, const int4* __restrict__ chunks, con
         {
             nlj += typeLJ[type[cd.x * kClusterSize + i]];
         }
-        cost[m] = cd.w * (kCostTile + (3 * nlj) / 2) + kCostChunk;
+        cost[m] = cd.w * (kCostTile + (3 * nlj) / 2) + chunkCost;
     }
 }
 
 // Share of the work given to each resident generation of workgroups.  The
 // dispatcher places workgroup b on CU b mod numCU, so with two workgroups
 // per CU the first numCU workgroups share every SIMD with the second ones;
-// the SIMD's arbiter issues for the older wavefront first, and at equal
-// work the second generation measured 9% slower, so the first generation
-// takes (1 + skew) and the second (1 - skew) of the average.  Other numbers
+// the SIMD's arbiter issues for the older wavefront first and the second
+// generation runs slower, so the first generation takes (1 + skew) and the
+// second (1 - skew) of the average.  Forces-only launch of the 288,000-atom
+// water box at a skew of 2.5, 4.5, 6.5, 8.5, 10.5 and 13 %: 163.5, 161.0,
+// 158.9, 157.8, 157.9 and 161.2 us; 150,000-atom chains 157, 153, 150.4,
+// 150.8, 151.0 and 158 us.  Other numbers
 // of generations are not weighted (not measured).  Returns the cumulative
 // weight of wavefronts [0, w) in 1/1000.
 __device__ long long generationWeight(int w, int numWaves, int genWaves)
@@ -1155,11 +1158,12 @@ void launchWaveSchedule(hipStream_t s, int numWaves, int nchunk, const int4* chu
                                                    costOff, costTotal, genWaves, out);
 }
 
-void launchChunkCosts(hipStream_t s, int nchunk, const int4* chunks, const int* type, const int* typeLJ, int* cost)
+void launchChunkCosts(hipStream_t s, int nchunk, const int4* chunks, const int* type, const int* typeLJ, int chunkCost,
+                      int* cost)
 {
     if (nchunk > 0)
     {
-        chunkCostKernel<<<(nchunk + 255) / 256, 256, 0, s>>>(nchunk, chunks, type, typeLJ, cost);
+        chunkCostKernel<<<(nchunk + 255) / 256, 256, 0, s>>>(nchunk, chunks, type, typeLJ, chunkCost, cost);
     }
 }
 

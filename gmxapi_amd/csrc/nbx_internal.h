@@ -61,13 +61,17 @@ constexpr int kGroupMaxJ    = 4096;
 constexpr int kTileJ        = 16;
 constexpr int kChunkEntries = 1 << 20;
 // cost of one chunk (i-entry) in work entries for the static schedule: its
-// i-data set-up and i-force reduction
-constexpr int kChunkWeight = 8;
+// i-data set-up and i-force reduction (64 replicas of 3,000 to 48,000 atoms:
+// 1016, 939 and 980 us per step with 8, 14 and 32)
+constexpr int kChunkWeight = 14;
+// the same for the adjoint's schedule (24,000-atom Hessian-vector product:
+// 85.2 us with 8, 86.6 with 14)
+constexpr int kAdjointChunkWeight = 8;
 // chunk cost model of the static schedule (1/32 tile) and the extra share of
 // the first resident generation of workgroups (1/1000)
 constexpr int kCostTile            = 32;
 constexpr int kCostChunk           = 27;
-constexpr int kGenerationSkewMilli = 45;
+constexpr int kGenerationSkewMilli = 80;
 // wavefronts per nonbonded workgroup, and the LDS a workgroup may use (two
 // resident workgroups per CU of 160 KiB, eight wavefronts); the adjoint may
 // use a CU's whole LDS
@@ -380,8 +384,14 @@ void launchWaveSchedule(hipStream_t s, int numWaves, int nchunk, const int4* chu
                         int ngroups, const int4* groups, int2* out, const int* costOff = nullptr,
                         const int* costTotal = nullptr, int genWaves = 0);
 // Per-chunk pair-kernel cost (1/32 tile units) from its tiles and the LJ
-// i-atoms of its cluster: type per cluster slot, typeLJ per type.
-void launchChunkCosts(hipStream_t s, int nchunk, const int4* chunks, const int* type, const int* typeLJ, int* cost);
+// i-atoms of its cluster (type per cluster slot, typeLJ per type), plus
+// chunkCost per chunk.  scheduleCostBound: at least the costs' total.
+void launchChunkCosts(hipStream_t s, int nchunk, const int4* chunks, const int* type, const int* typeLJ, int chunkCost,
+                      int* cost);
+inline long long scheduleCostBound(int nwork, int nchunk, int chunkCost)
+{
+    return static_cast<long long>(nwork / kTileJ + 1) * (kCostTile + 6) + static_cast<long long>(chunkCost) * nchunk;
+}
 // Energy-slot range of each system of a batch: slotOff[k] for k in [0, R]
 // (the kernel's slot g + w of the first chunk of the system's first group).
 void launchSystemSlots(hipStream_t s, int numSystems, const int* groupOff, int ngroups, const int4* groups,

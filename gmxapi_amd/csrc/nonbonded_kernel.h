@@ -67,7 +67,8 @@
 // fma(fma(rinv, rinv, -F), qq rinv, LJ), the masked 1/r put pairs beyond the
 // cut-off on the table's first entry and the window update lost its branch).
 // 288,000-atom water, table Ewald: forces only 184 -> 164 us, with energies
-// and shift forces 210 -> 197 us; 150,000-atom chains 174 -> 157 us.
+// and shift forces 210 -> 197 us; 150,000-atom chains 174 -> 157 us.  The
+// start-up reads in flight together took 2 us more off every launch.
 // The code is a header so that each Coulomb flavour's instantiations compile
 // in a source file of their own (kernel_rf.hip, kernel_table.hip,
 // kernel_analytical.hip).
@@ -363,6 +364,53 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     float4*         sTab   = smem4 + L.tab;
     float*          sFsh   = reinterpret_cast<float*>(smem4 + L.fsh);
 
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x / kWave;
+    const int jj   = lane & 3;
+    const int kk   = lane >> 2;
+
+    // The start-up's reads are in flight together: the Ewald table's, and down
+    // the chain from this wavefront's run (its chunks, balanced by cost when
+    // the list was built) to its first work entries and j-atoms.  One after
+    // the other they cost 2 to 3 us of every launch.
+    const int  wid   = blockIdx.x * kWavesBlock + wave;
+    const int2 ws    = a.waveStart[wid];
+    const int  wsEnd = a.waveStart[wid + 1].x;
+    // the energy kernels' table starts with an entry of zeros; without
+    // energies only {F, dF} are kept, half the LDS banks per read
+    auto tableEntry = [&](int t) { return a.tabFDV0[kEnergy ? max(t - 1, 0) : min(t, tabN - 2)]; };
+    auto storeEntry = [&](int t, const float4 v) {
+        if (kEnergy)
+        {
+            sTab[t] = t > 0 ? v : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+        else
+        {
+            reinterpret_cast<float2*>(sTab)[t] = make_float2(v.x, v.y);
+        }
+    };
+    constexpr int kTabRegs = kElec == kElecEwaldTable ? 5 : 0;
+    float4        tabReg[kTabRegs + 1];
+#pragma unroll
+    for (int k = 0; k < kTabRegs; k++)
+    {
+        const int t = threadIdx.x + k * kThreads;
+        tabReg[k]   = tableEntry(min(t, tabN - 1));
+    }
+    const int chAll0 = uniformInt(ws.x);
+    const int chAll1 = uniformInt(wsEnd);
+    const int gFirst = uniformInt(ws.y);
+    int4      cFirst = make_int4(0, 0, 0, 0), cLast = cFirst, grpFirst = cFirst, infoFirst = cFirst, segFirst = cFirst;
+    float4    shiftFirst = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (chAll0 < chAll1)
+    {
+        cFirst     = a.chunks[chAll0];
+        cLast      = a.chunks[chAll1 - 1];
+        shiftFirst = a.chunkShift[chAll0];
+        grpFirst   = a.groups[gFirst];
+        infoFirst  = a.groupInfo[gFirst];
+        segFirst   = a.segInfo[gFirst];
+    }
     for (int t = threadIdx.x; t < ntype2; t += kThreads)
     {
         sNbfp[t] = a.nbfp[t];
@@ -374,54 +422,51 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             sC6g[t] = a.c6grid[t];
         }
     }
-    for (int t = threadIdx.x; t < tabN; t += kThreads)
-    {
-        if (kEnergy)
-        {
-            sTab[t] = t > 0 ? a.tabFDV0[t - 1] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-        else
-        {
-            // without energies only {F, dF}: half the LDS banks per read
-            const float4 v = a.tabFDV0[min(t, tabN - 2)];
-            reinterpret_cast<float2*>(sTab)[t] = make_float2(v.x, v.y);
-        }
-    }
     // one shift-force array per wavefront: each is summed in the wavefront's
     // own (fixed) order, and the four are added in wavefront order at the end
     for (int t = threadIdx.x; t < kWavesBlock * kNumShifts * 3; t += kThreads)
     {
         sFsh[t] = 0.0f;
     }
+    // the run is walked by one software pipeline, across i-entry and group
+    // boundaries; reads past its last tile are clamped to it
+    const unsigned W0 = static_cast<unsigned>(uniformInt(cFirst.z));
+    const int      T  = (uniformInt(cLast.z) - static_cast<int>(W0)) / kTileJ + uniformInt(cLast.w);
+    auto entryAt      = [&](int t) {
+        return ldg(a.work, W0 + static_cast<unsigned>(kTileJ * min(t, T - 1) + kk));
+    };
+    uint2 e0 = make_uint2(0u, 0u), e1 = e0, e2 = e0, e3 = e0;
+    if (chAll0 < chAll1)
+    {
+        e0 = entryAt(0);
+        e1 = entryAt(1);
+        e2 = entryAt(2);
+        e3 = entryAt(3);
+    }
+#pragma unroll
+    for (int k = 0; k < kTabRegs; k++)
+    {
+        const int t = threadIdx.x + k * kThreads;
+        if (t < tabN)
+        {
+            storeEntry(t, tabReg[k]);
+        }
+    }
+    for (int t = threadIdx.x + kTabRegs * kThreads; t < tabN; t += kThreads)
+    {
+        storeEntry(t, tableEntry(t));
+    }
     __syncthreads();
-
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    const int jj   = lane & 3;
-    const int kk   = lane >> 2;
 
     const InteractionConst ic = a.ic;
     // this wavefront's j-force window
     float* win = reinterpret_cast<float*>(smem4 + L.win) + wave * a.windowSlots * 12;
 
-    // this wavefront's contiguous run of chunks (balanced by cost when the
-    // list was built); chunks and work entries are stored in group order, so
-    // one software pipeline runs over the whole run, across i-entry and group
-    // boundaries
-    const int  wid    = blockIdx.x * kWavesBlock + wave;
-    const int2 ws     = a.waveStart[wid];
-    const int  chAll0 = uniformInt(ws.x);
-    const int  chAll1 = uniformInt(a.waveStart[wid + 1].x);
     if (chAll0 < chAll1)
     {
-        const int4     cFirst = a.chunks[chAll0];
-        const int4     cLast  = a.chunks[chAll1 - 1];
-        const unsigned W0     = static_cast<unsigned>(uniformInt(cFirst.z));
-        const int      T      = (uniformInt(cLast.z) - static_cast<int>(W0)) / kTileJ + uniformInt(cLast.w);
-
         // current group (the run starts inside the group holding its first
         // chunk); wavefront w writes the energies of group g to slot g + w
-        int g = uniformInt(ws.y), chGrpEnd = 0, U = 0, c0 = 0, G = 0, stage = -1;
+        int g = gFirst, chGrpEnd = 0, U = 0, c0 = 0, G = 0, stage = -1;
         // current chunk
         IAtoms I;
         float4 sv;
@@ -434,10 +479,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         bool   central = false;
         double eVdw = 0.0, eCoul = 0.0;
 
-        auto beginGroup = [&](int gg) {
-            const int4 grp = a.groups[gg]; // chunk range, union offset, windowed union size
-            const int4 gi  = a.groupInfo[gg]; // first own cluster, own count | G << 16
-            const int4 si  = a.segInfo[gg];   // staging: first float4, first wavefront, wavefronts, size
+        // grp: chunk range, union offset, windowed union size; gi: first own
+        // cluster, own count | G << 16; si: the staging's first float4, first
+        // wavefront, wavefronts, size
+        auto beginGroup = [&](const int4 grp, const int4 gi, const int4 si) {
             chGrpEnd       = uniformInt(grp.y);
             U              = uniformInt(grp.w);
             c0             = uniformInt(gi.x);
@@ -596,27 +641,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             {
                 endGroup();
                 g++;
-                beginGroup(g);
+                beginGroup(a.groups[g], a.groupInfo[g], a.segInfo[g]);
             }
             beginChunk(cdNext, svNext, t);
             cdNext = a.chunks[min(chIdx + 1, chAll1 - 1)];
             svNext = a.chunkShift[min(chIdx + 1, chAll1 - 1)];
         };
 
-        // reads past the last tile are clamped to it
-        auto entryAt = [&](int t) {
-            return ldg(a.work, W0 + static_cast<unsigned>(kTileJ * min(t, T - 1) + kk));
-        };
         auto loadX = [&](const uint2 e) { return ldg(a.xq, e.x * kClusterSize + jj); };
         auto loadT = [&](const uint2 e) { return ldg(a.type, e.x * kClusterSize + jj); };
         // tiles t and t + 1 (entries, j-atoms), entries of t + 2 and t + 3
-        uint2  e0 = entryAt(0), e1 = entryAt(1), e2 = entryAt(2), e3 = entryAt(3);
         float4 x0 = loadX(e0);
         int    y0 = loadT(e0);
         float4 x1 = loadX(e1);
         int    y1 = loadT(e1);
-        beginGroup(g);
-        beginChunk(cFirst, a.chunkShift[chAll0], 0);
+        beginGroup(grpFirst, infoFirst, segFirst);
+        beginChunk(cFirst, shiftFirst, 0);
         // an odd tile count: the first tile alone, so that the loop below
         // always runs whole pairs of tiles (with no exit between its two
         // tiles the compiler keeps the accumulators in place: about 14 register
