@@ -21,9 +21,10 @@
 // first j entry of every central i-entry.
 //
 // Work decomposition: one wavefront per i-cluster; lanes take one candidate
-// cluster each, hits are compacted in candidate order with a ballot, so the
-// output is deterministic.  The same kernel runs twice: a count pass (per
+// cluster each, candidates and hits are compacted in candidate order with
+// ballots, so the output is deterministic.  The same kernel runs twice: a count pass (per
 // i-cluster j and i counts, scanned on the device) and a fill pass.
+#include <cfloat>
 #include <cstdint>
 
 #include "nbx_internal.h"
@@ -74,73 +75,103 @@ __device__ __forceinline__ int wavePrefixExclusive(int v, int lane, int* total)
     return x - v;
 }
 
-// The first m in [s, e) with pred(m) true (e if none) for a predicate that
-// is false then true along the range: up to three probes stepping from the
-// guess (an exact guess settles in two), then bisection of what is left.
-template<typename P>
-__device__ __forceinline__ int firstTrue(int s, int e, int guess, P pred)
+// A wavefront's candidates of one window of columns, and the ones whose
+// bounding boxes are in range, waiting for their atom distances (LDS)
+constexpr int kCandidates = 512;
+constexpr int kWaiting    = 2 * kWave;
+
+// Orders a wavefront's own LDS accesses for the compiler (the hardware keeps
+// a wavefront's LDS accesses in order).
+__device__ __forceinline__ void waveLdsFence()
 {
-    int lo = s, hi = e; // the answer lies in [lo, hi]
-    int m  = min(max(guess, s), e - 1);
-    for (int it = 0; it < 3 && lo < hi && m >= lo && m < hi; it++)
-    {
-        if (pred(m))
-        {
-            hi = m;
-            m--;
-        }
-        else
-        {
-            lo = m + 1;
-            m++;
-        }
-    }
-    while (lo < hi)
-    {
-        const int mid = (lo + hi) >> 1;
-        if (pred(mid))
-        {
-            hi = mid;
-        }
-        else
-        {
-            lo = mid + 1;
-        }
-    }
-    return lo;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-template<bool kFill>
-__global__ __launch_bounds__(kWave* kSearchWaves) void searchKernel(SearchArgs a)
+// A wave-uniform float in a scalar register
+__device__ __forceinline__ float uniformF(float v)
 {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+// One probe of two bounds searched side by side: [lo, hi] holds the first m
+// with the predicate true (t: its value at m), the next probe a neighbour of
+// this one for the first two (they start at a guess), then the middle.
+__device__ __forceinline__ void boundStep(bool t, int probe, int& lo, int& hi, int& m)
+{
+    if (t)
+    {
+        hi = m;
+        m--;
+    }
+    else
+    {
+        lo = m + 1;
+        m++;
+    }
+    if (probe >= 2 || m < lo || m >= hi)
+    {
+        m = (lo + hi) >> 1;
+    }
+}
+
+// What bounds it: latency and VALU issue about evenly (a dozen dependent
+// reads per cluster; 1,340 VALU instructions per cluster on 288,000-atom water,
+// 2,200 before).  The cluster is wave-uniform, so its boxes and atoms sit in
+// scalar registers and five wavefronts fit a SIMD (four or eight, the latter
+// with spills, measured 6 and 20 us slower).  Only the shifts that can reach the box are
+// walked (one for most clusters, not 14).  A column's candidates end where
+// the sphere of radius rlist around the i-cluster's bounding box leaves the
+// column; both ends are searched at once.  Candidates in bounding-box range
+// are collected before their distances are taken, so those run on full
+// wavefronts, and the distances are fused multiply-adds: only a smallest one
+// within 1e-6 of rlist^2 (the two roundings differ by less than 6 * 2^-24) is
+// taken again with the canonical rounding, which decides.
+// 288,000-atom water: 410 -> 245 us.
+template<bool kFill>
+__global__ __launch_bounds__(kWave* kSearchWaves) __attribute__((amdgpu_waves_per_eu(5))) void searchKernel(SearchArgs a)
+{
+    __shared__ int sCand[kSearchWaves][kCandidates];
+    __shared__ int sWait[kSearchWaves][kWaiting];
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int ci   = blockIdx.x * kSearchWaves + wave;
     if (ci >= a.ncluster)
     {
         return;
     }
-    const GridDims& g = a.g;
-    const float4 bbLo = a.bb[2 * ci];
-    const float4 bbHi = a.bb[2 * ci + 1];
-    float4 xi[kClusterSize];
-    int    iIndexReal[kClusterSize];
+    int* const      cand = sCand[wave];
+    int* const      wait = sWait[wave];
+    const GridDims& g    = a.g;
+    const float4    lo   = a.bb[2 * ci], hi = a.bb[2 * ci + 1];
+    float4          xi[kClusterSize];
+    int             iIndexReal[kClusterSize];
 #pragma unroll
     for (int i = 0; i < kClusterSize; i++)
     {
         xi[i]         = a.xq[ci * kClusterSize + i];
         iIndexReal[i] = a.atomIndices[ci * kClusterSize + i];
+        if (iIndexReal[i] < 0)
+        {
+            // far from every atom and from the j-clusters' fillers
+            xi[i].x = xi[i].y = xi[i].z = -3.0f * kFarAway;
+        }
+        xi[i].x = uniformF(xi[i].x);
+        xi[i].y = uniformF(xi[i].y);
+        xi[i].z = uniformF(xi[i].z);
     }
-    const float rl     = a.rlist;
-    const float rlist2 = a.rlist2;
+    const float rl      = a.rlist;
+    const float rlist2  = a.rlist2;
+    const float inside  = rlist2 * (1.0f - 1e-6f);
+    const float outside = rlist2 * (1.0f + 1e-6f);
 
     int jpos = 0, ipos = 0;
     // fill pass: the i-cluster's topology exclusions (other than an atom
     // with itself), one per lane: the excluded atom's slot and the i-atom's
     // index in the cluster; numExcl is wave-uniform.  Every hit's mask is
-    // then built from these with shuffles instead of walking the exclusion
-    // lists per candidate.  More than a wavefront's worth (not seen for
-    // bonded exclusions) falls back to the walk.
+    // then built from these, read lane by lane into scalar registers, instead
+    // of walking the exclusion lists per candidate.  More than a wavefront's
+    // worth (not seen for bonded exclusions) falls back to the walk.
     int numExcl = 0, exSlot = -1, exI = 0;
     if (kFill)
     {
@@ -158,6 +189,7 @@ __global__ __launch_bounds__(kWave* kSearchWaves) void searchKernel(SearchArgs a
             cnt[i]          = iAtom >= 0 ? a.exclOff[iAtom + 1] - beg[i] : 0;
             numExcl += cnt[i];
         }
+        numExcl = __builtin_amdgcn_readfirstlane(numExcl);
         if (numExcl <= kWave)
         {
             int base = 0;
@@ -175,12 +207,24 @@ __global__ __launch_bounds__(kWave* kSearchWaves) void searchKernel(SearchArgs a
         }
     }
     int countJ = 0, countI = 0;
+    const float4 bbLo = make_float4(uniformF(lo.x), uniformF(lo.y), uniformF(lo.z), 0.0f);
+    const float4 bbHi = make_float4(uniformF(hi.x), uniformF(hi.y), uniformF(hi.z), 0.0f);
+    // the shifts that leave the box within rlist of the cell, per direction
+    // (most clusters have the central one only): shift +1 is out of range
+    // when the shifted lower bound lies beyond rlist of the upper face, -1
+    // when the shifted upper bound lies beyond rlist below the lower one
+    const bool up[3]   = { !(uniformF(__fadd_rn(bbLo.x, g.box[0]) - rl) > g.box[0]),
+                           !(uniformF(__fadd_rn(bbLo.y, g.box[1]) - rl) > g.box[1]), true };
+    const bool down[3] = { !(uniformF(__fadd_rn(bbHi.x, -g.box[0]) + rl) < 0.0f),
+                           !(uniformF(__fadd_rn(bbHi.y, -g.box[1]) + rl) < 0.0f),
+                           !(uniformF(__fadd_rn(bbHi.z, -g.box[2]) + rl) < 0.0f) };
 
-    for (int tz = -1; tz <= 1; tz++)
+    // shifts up to the central one: no z shift up
+    for (int tz = down[2] ? -1 : 0; tz <= 0; tz++)
     {
-        for (int ty = -1; ty <= 1; ty++)
+        for (int ty = down[1] ? -1 : 0; ty <= (up[1] ? 1 : 0); ty++)
         {
-            for (int tx = -1; tx <= 1; tx++)
+            for (int tx = down[0] ? -1 : 0; tx <= (up[0] ? 1 : 0); tx++)
             {
                 const int shift = xyz2is(tx, ty, tz);
                 if (shift > kCentral)
@@ -192,15 +236,21 @@ __global__ __launch_bounds__(kWave* kSearchWaves) void searchKernel(SearchArgs a
                 const float shy = static_cast<float>(ty) * g.box[1];
                 const float shz = static_cast<float>(tz) * g.box[2];
                 // set_icell_bb_simple: shifted i bounding box
-                const float4 lo4 = make_float4(__fadd_rn(bbLo.x, shx), __fadd_rn(bbLo.y, shy), __fadd_rn(bbLo.z, shz), 0);
-                const float4 hi4 = make_float4(__fadd_rn(bbHi.x, shx), __fadd_rn(bbHi.y, shy), __fadd_rn(bbHi.z, shz), 0);
+                const float4 lo4 = make_float4(uniformF(__fadd_rn(bbLo.x, shx)), uniformF(__fadd_rn(bbLo.y, shy)),
+                                               uniformF(__fadd_rn(bbLo.z, shz)), 0);
+                const float4 hi4 = make_float4(uniformF(__fadd_rn(bbHi.x, shx)), uniformF(__fadd_rn(bbHi.y, shy)),
+                                               uniformF(__fadd_rn(bbHi.z, shz)), 0);
                 // conservative column and z ranges (margin 1% of a cell)
                 if (lo4.x - rl > g.box[0] || hi4.x + rl < 0 || lo4.y - rl > g.box[1] || hi4.y + rl < 0
                     || lo4.z - rl > g.box[2] || hi4.z + rl < 0)
                 {
                     continue;
                 }
-                const int cxf = max(0, static_cast<int>(floorf((lo4.x - rl) * g.invCellSize[0] - 0.01f)));
+                // (centrally the clusters before ci are left out, and with
+                // them the columns before its own)
+                const float xFirst = central ? lo4.x : lo4.x - rl;
+                const int cxf =
+                        min(max(0, static_cast<int>(floorf(xFirst * g.invCellSize[0] - 0.01f))), g.ncx - 1);
                 const int cxl = min(g.ncx - 1, static_cast<int>(floorf((hi4.x + rl) * g.invCellSize[0] + 0.01f)));
                 const int cyf = max(0, static_cast<int>(floorf((lo4.y - rl) * g.invCellSize[1] - 0.01f)));
                 const int cyl = min(g.ncy - 1, static_cast<int>(floorf((hi4.y + rl) * g.invCellSize[1] + 0.01f)));
@@ -208,20 +258,118 @@ __global__ __launch_bounds__(kWave* kSearchWaves) void searchKernel(SearchArgs a
                 {
                     continue;
                 }
-                const float zlo = lo4.z - rl - 1e-3f;
-                const float zhi = hi4.z + rl + 1e-3f;
                 float xs[kClusterSize], ys[kClusterSize], zs[kClusterSize];
 #pragma unroll
                 for (int i = 0; i < kClusterSize; i++)
                 {
-                    xs[i] = __fadd_rn(xi[i].x, shx);
-                    ys[i] = __fadd_rn(xi[i].y, shy);
-                    zs[i] = __fadd_rn(xi[i].z, shz);
+                    xs[i] = uniformF(__fadd_rn(xi[i].x, shx));
+                    ys[i] = uniformF(__fadd_rn(xi[i].y, shy));
+                    zs[i] = uniformF(__fadd_rn(xi[i].z, shz));
                 }
                 const int nyc      = cyl - cyf + 1;
                 const int numCols  = (cxl - cxf + 1) * nyc;
                 int       entryJ   = 0; // j entries of this (ci, shift)
                 const int entryPos = jpos + countJ;
+                int       waiting  = 0;
+                // the first n waiting candidates: atom distances, exclusion
+                // masks, and the hits written in candidate order
+                auto takeWaiting = [&](int n) {
+                    const int cj  = wait[min(lane, n - 1)];
+                    bool      hit = false;
+                    if (lane < n)
+                    {
+                        float least = FLT_MAX;
+#pragma unroll
+                        for (int j = 0; j < kClusterSize; j++)
+                        {
+                            const float4 xj = a.xq[cj * kClusterSize + j];
+#pragma unroll
+                            for (int i = 0; i < kClusterSize; i++)
+                            {
+                                const float dx = __fsub_rn(xs[i], xj.x), dy = __fsub_rn(ys[i], xj.y),
+                                            dz = __fsub_rn(zs[i], xj.z);
+                                least          = fminf(least, fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
+                            }
+                        }
+                        hit = least < inside || (central && cj == ci);
+                        if (!hit && least < outside)
+                        {
+#pragma unroll 1
+                            for (int j = 0; j < kClusterSize; j++)
+                            {
+                                const float4 xj = a.xq[cj * kClusterSize + j];
+#pragma unroll
+                                for (int i = 0; i < kClusterSize; i++)
+                                {
+                                    hit = hit
+                                          || canonicalD2(__fsub_rn(xs[i], xj.x), __fsub_rn(ys[i], xj.y),
+                                                         __fsub_rn(zs[i], xj.z))
+                                                     < rlist2;
+                                }
+                            }
+                        }
+                    }
+                    const unsigned long long ballot = __ballot(hit);
+                    const int                before = __popcll(ballot & ((1ull << lane) - 1ull));
+                    // a capped region past its end: not written, the
+                    // count (above capJ) sends the host to the counted path
+                    const bool room = a.capJ == 0 || entryPos + entryJ + before < jpos + a.capJ;
+                    if (kFill && ballot != 0 && numExcl <= kWave)
+                    {
+                        // exclusion bits 4 i + j of the exclusions in this
+                        // j-cluster (setExclusionsForIEntry,
+                        // pairlist.cpp:1367-1435); centrally a pair is
+                        // excluded only in the entry of its lower slot
+                        unsigned exclMask = 0u;
+                        for (int k = 0; k < numExcl; k++)
+                        {
+                            const int js = __builtin_amdgcn_readlane(exSlot, k);
+                            const int ii = __builtin_amdgcn_readlane(exI, k);
+                            if (js >= 0 && !(central && js <= ci * kClusterSize + ii))
+                            {
+                                const unsigned bit = 1u << (ii * kClusterSize + (js & 3));
+                                exclMask |= (js >> 2) == cj ? bit : 0u;
+                            }
+                        }
+                        if (hit && room)
+                        {
+                            const unsigned mask = ((central && cj == ci) ? kMaskDiag : kMaskAll) & ~exclMask;
+                            a.jentry[entryPos + entryJ + before] = make_uint2(static_cast<unsigned>(cj), mask);
+                        }
+                    }
+                    else if (kFill && hit && room)
+                    {
+                        unsigned mask = (central && cj == ci) ? kMaskDiag : kMaskAll;
+                        for (int i = 0; i < kClusterSize; i++)
+                        {
+                            const int iAtom = iIndexReal[i];
+                            if (iAtom < 0)
+                            {
+                                continue;
+                            }
+                            const int iIndex = ci * kClusterSize + i;
+                            for (int k = a.exclOff[iAtom]; k < a.exclOff[iAtom + 1]; k++)
+                            {
+                                const int jAtom = a.exclIdx[k];
+                                if (jAtom == iAtom)
+                                {
+                                    continue;
+                                }
+                                const int jIndex = a.cells[jAtom];
+                                if (central && jIndex <= iIndex)
+                                {
+                                    continue;
+                                }
+                                if ((jIndex >> 2) == cj)
+                                {
+                                    mask &= ~(1u << (i * kClusterSize + (jIndex & 3)));
+                                }
+                            }
+                        }
+                        a.jentry[entryPos + entryJ + before] = make_uint2(static_cast<unsigned>(cj), mask);
+                    }
+                    entryJ += __popcll(ballot);
+                };
                 for (int c0 = 0; c0 < numCols; c0 += kWave)
                 {
                     // per-lane column: z range of candidate clusters
@@ -232,143 +380,97 @@ __global__ __launch_bounds__(kWave* kSearchWaves) void searchKernel(SearchArgs a
                         const int cx  = cxf + cc / nyc;
                         const int cy  = cyf + cc % nyc;
                         const int col = cx * g.ncy + cy;
-                        int       s   = a.cxy_ind[col];
-                        int       e   = a.cxy_ind[col + 1];
-                        // the column's clusters are sorted by z (both bounds
-                        // non-decreasing): the first with upper z >= zlo and
-                        // the first with lower z > zhi, each searched from
-                        // where an even spread over the box height puts it
-                        const float perZ  = static_cast<float>(e - s) * g.invBoxZ;
-                        const int   first = firstTrue(s, e, s + static_cast<int>(zlo * perZ),
-                                                      [&](int m) { return a.bb[2 * m + 1].z >= zlo; });
-                        int last = firstTrue(first, e, s + static_cast<int>(zhi * perZ) + 1,
-                                             [&](int m) { return a.bb[2 * m].z > zhi; }); // exclusive
-                        k0       = first;
-                        if (central)
+                        const int s   = a.cxy_ind[col];
+                        const int e   = a.cxy_ind[col + 1];
+                        // the sphere's half height over the column, from the
+                        // box's distance to it (margin 1% of a cell; the
+                        // outermost columns are open outwards)
+                        const float mx = 0.01f * g.cellSize[0], my = 0.01f * g.cellSize[1];
+                        const float cl = cx > 0 ? cx * g.cellSize[0] - mx - hi4.x : 0.0f;
+                        const float ch = cx < g.ncx - 1 ? lo4.x - ((cx + 1) * g.cellSize[0] + mx) : 0.0f;
+                        const float rl_ = cy > 0 ? cy * g.cellSize[1] - my - hi4.y : 0.0f;
+                        const float rh  = cy < g.ncy - 1 ? lo4.y - ((cy + 1) * g.cellSize[1] + my) : 0.0f;
+                        const float dx = fmaxf(fmaxf(cl, ch), 0.0f), dy = fmaxf(fmaxf(rl_, rh), 0.0f);
+                        const float h2 = rl * rl * (1.0f + 1e-5f) - dx * dx - dy * dy;
+                        if (h2 > 0.0f && s < e)
                         {
-                            k0 = max(k0, ci);
+                            const float h   = sqrtf(h2) + 1e-3f;
+                            const float zlo = lo4.z - h;
+                            const float zhi = hi4.z + h;
+                            // the column's clusters are sorted by z (both bounds
+                            // non-decreasing): the first with upper z >= zlo and
+                            // the first with lower z > zhi (exclusive end), both
+                            // searched at once, each from where an even spread
+                            // over the box height puts it
+                            const float perZ = static_cast<float>(e - s) * g.invBoxZ;
+                            int         lo0 = s, hi0 = e, lo1 = s, hi1 = e;
+                            int         m0 = min(max(s + static_cast<int>(zlo * perZ), s), e - 1);
+                            int         m1 = min(max(s + static_cast<int>(zhi * perZ) + 1, s), e - 1);
+                            for (int probe = 0; lo0 < hi0 || lo1 < hi1; probe++)
+                            {
+                                const float z0 = a.bb[2 * min(m0, e - 1) + 1].z;
+                                const float z1 = a.bb[2 * min(m1, e - 1)].z;
+                                if (lo0 < hi0)
+                                {
+                                    boundStep(z0 >= zlo, probe, lo0, hi0, m0);
+                                }
+                                if (lo1 < hi1)
+                                {
+                                    boundStep(z1 > zhi, probe, lo1, hi1, m1);
+                                }
+                            }
+                            k0 = central ? max(lo0, ci) : lo0;
+                            n  = max(0, lo1 - k0);
                         }
-                        n = max(0, last - k0);
                     }
-                    int total;
-                    const int pref     = wavePrefixExclusive(n, lane, &total);
-                    const int ncolHere = min(kWave, numCols - c0);
-                    for (int t0 = 0; t0 < total; t0 += kWave)
+                    int       total;
+                    const int pref = wavePrefixExclusive(n, lane, &total);
+                    for (int w0 = 0; w0 < total; w0 += kCandidates)
                     {
-                        const int t = t0 + lane;
-                        // column slot holding candidate t: the last slot whose
-                        // prefix is <= t (uniform trip count, all lanes shuffle)
-                        int lo = 0, hiIdx = ncolHere - 1;
-#pragma unroll
-                        for (int it = 0; it < 7; it++)
+                        // the candidates [w0, w0 + kCandidates) in column order
+                        const int kEnd = min(n, w0 + kCandidates - pref);
+                        int       k    = max(0, w0 - pref);
+                        waveLdsFence();
+                        for (; __any(k < kEnd); k++)
                         {
-                            const int m  = (lo + hiIdx + 1) >> 1;
-                            const int pm = __shfl(pref, m, kWave);
-                            if (lo < hiIdx)
+                            if (k < kEnd)
                             {
-                                if (pm <= t)
-                                {
-                                    lo = m;
-                                }
-                                else
-                                {
-                                    hiIdx = m - 1;
-                                }
+                                cand[pref + k - w0] = k0 + k;
                             }
                         }
-                        const int colStart = __shfl(k0, lo, kWave);
-                        const int colPref  = __shfl(pref, lo, kWave);
-                        bool      hit      = false;
-                        int       cj       = -1;
-                        if (t < total)
+                        waveLdsFence();
+                        const int here = min(kCandidates, total - w0);
+                        for (int t0 = 0; t0 < here; t0 += kWave)
                         {
-                            cj = colStart + (t - colPref);
-                            if (central && cj == ci)
+                            const int t    = t0 + lane;
+                            const int cj   = cand[min(t, here - 1)];
+                            bool      near = false;
+                            if (t < here)
                             {
-                                hit = true;
+                                near = bbDist2(lo4, hi4, a.bb[2 * cj], a.bb[2 * cj + 1]) < rlist2;
                             }
-                            else
+                            const unsigned long long ballot = __ballot(near);
+                            if (near)
                             {
-                                const float4 jlo = a.bb[2 * cj];
-                                const float4 jhi = a.bb[2 * cj + 1];
-                                if (bbDist2(lo4, hi4, jlo, jhi) < rlist2)
-                                {
-#pragma unroll
-                                    for (int j = 0; j < kClusterSize; j++)
-                                    {
-                                        const float4 xj = a.xq[cj * kClusterSize + j];
-#pragma unroll
-                                        for (int i = 0; i < kClusterSize; i++)
-                                        {
-                                            const float d2 = canonicalD2(__fsub_rn(xs[i], xj.x), __fsub_rn(ys[i], xj.y),
-                                                                     __fsub_rn(zs[i], xj.z));
-                                            hit = hit || (iIndexReal[i] >= 0 && d2 < rlist2);
-                                        }
-                                    }
-                                }
+                                wait[waiting + __popcll(ballot & ((1ull << lane) - 1ull))] = cj;
+                            }
+                            waiting += __popcll(ballot);
+                            waveLdsFence();
+                            if (waiting >= kWave)
+                            {
+                                takeWaiting(kWave);
+                                const int rest = wait[kWave + lane];
+                                waveLdsFence();
+                                wait[lane] = rest;
+                                waiting -= kWave;
+                                waveLdsFence();
                             }
                         }
-                        const unsigned long long ballot = __ballot(hit);
-                        const int before = __popcll(ballot & ((1ull << lane) - 1ull));
-                        // exclusion bits 4 i + j of the exclusions in this
-                        // j-cluster (setExclusionsForIEntry,
-                        // pairlist.cpp:1367-1435), every lane taking part in
-                        // the shuffles; centrally a pair is excluded only in
-                        // the entry of its lower slot
-                        unsigned exclMask = 0u;
-                        if (kFill && ballot != 0 && numExcl <= kWave)
-                        {
-                            for (int k = 0; k < numExcl; k++)
-                            {
-                                const int js = __shfl(exSlot, k, kWave);
-                                const int ii = __shfl(exI, k, kWave);
-                                if (js >= 0 && (js >> 2) == cj && !(central && js <= ci * kClusterSize + ii))
-                                {
-                                    exclMask |= 1u << (ii * kClusterSize + (js & 3));
-                                }
-                            }
-                        }
-                        // a capped region past its end: not written, the
-                        // count (above capJ) sends the host to the counted path
-                        const bool room = a.capJ == 0 || entryPos + entryJ + before < jpos + a.capJ;
-                        if (kFill && hit && room && numExcl <= kWave)
-                        {
-                            const unsigned mask = ((central && cj == ci) ? kMaskDiag : kMaskAll) & ~exclMask;
-                            a.jentry[entryPos + entryJ + before] = make_uint2(static_cast<unsigned>(cj), mask);
-                        }
-                        else if (kFill && hit && room)
-                        {
-                            unsigned mask = (central && cj == ci) ? kMaskDiag : kMaskAll;
-                            for (int i = 0; i < kClusterSize; i++)
-                            {
-                                const int iAtom = iIndexReal[i];
-                                if (iAtom < 0)
-                                {
-                                    continue;
-                                }
-                                const int iIndex = ci * kClusterSize + i;
-                                for (int k = a.exclOff[iAtom]; k < a.exclOff[iAtom + 1]; k++)
-                                {
-                                    const int jAtom = a.exclIdx[k];
-                                    if (jAtom == iAtom)
-                                    {
-                                        continue;
-                                    }
-                                    const int jIndex = a.cells[jAtom];
-                                    if (central && jIndex <= iIndex)
-                                    {
-                                        continue;
-                                    }
-                                    if ((jIndex >> 2) == cj)
-                                    {
-                                        mask &= ~(1u << (i * kClusterSize + (jIndex & 3)));
-                                    }
-                                }
-                            }
-                            a.jentry[entryPos + entryJ + before] = make_uint2(static_cast<unsigned>(cj), mask);
-                        }
-                        entryJ += __popcll(ballot);
                     }
+                }
+                if (waiting > 0)
+                {
+                    takeWaiting(waiting);
                 }
                 if (entryJ > 0)
                 {
