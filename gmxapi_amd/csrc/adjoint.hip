@@ -15,7 +15,8 @@
 // stored per pair: the kernel walks the same work list, groups and static
 // schedule as the forward kernel and recomputes every pair.
 //
-// Mapping: as in the forward kernel, four wave-uniform i-atoms per tile and
+// Mapping: as in the forward kernel (its i-atoms through scalar loads and its
+// prefetch distances too), four wave-uniform i-atoms per tile and
 // one j-atom per lane.  A wavefront's LDS window holds {dL/dx, dL/dq} per
 // j-cluster atom (float4); i-atom sums live in 16 registers per i-entry and
 // are reduce-scattered once per entry.  Windows are staged with plain stores
@@ -23,7 +24,15 @@
 // summed in double there); the C6/C12 gradients are summed per workgroup in
 // LDS in double (ds_add_f64) and the workgroup sums are added in a fixed
 // order.
-// Two wavefronts per workgroup keep the float4 window of a workgroup small.
+// Four wavefronts per workgroup and two workgroups per CU: two wavefronts on
+// every SIMD.  (With two-wavefront workgroups three fitted a CU, and the two
+// SIMDs with two wavefronts each finished last.)  The first generation of
+// workgroups takes the larger share, as in the forward kernel's schedule.
+// What bounds it: VALU issue (about 75 instructions per pair) and the launch's
+// tail.  Hessian-vector product of the 24,000-atom chains (set-up and gather
+// included): 86 us; 84 with scalar i-atoms and the deeper prefetch, 73 with
+// two full generations, 70 with their shares, 68.7 with the four i-atoms'
+// arithmetic interleaved.
 #include "kernel_common.h"
 
 namespace nbx
@@ -32,21 +41,18 @@ namespace nbx
 namespace
 {
 
-constexpr int kAdjWaves   = 2;
+constexpr int kAdjWaves   = kAdjointWaves;
 constexpr int kAdjThreads = kWave * kAdjWaves;
 
 // LDS layout of an adjoint workgroup, in float4 units
 struct AdjLayout
 {
-    int nbfp, tab, ix, ig, it, win, acc, end_;
+    int nbfp, tab, win, acc, end_;
     __host__ __device__ AdjLayout(int ntype, int tabN, int windowSlots)
     {
         nbfp = 0;
         tab  = nbfp + (ntype * ntype + 1) / 2;
-        ix   = tab + tabN;
-        ig   = ix + kAdjWaves * kGroupSizeMax * kClusterSize;
-        it   = ig + kAdjWaves * kGroupSizeMax * kClusterSize;
-        win  = it + kAdjWaves * kGroupSizeMax;
+        win  = tab + tabN;
         acc  = win + kAdjWaves * windowSlots * 4;
         // {dC6, dC12} per type pair as two doubles, in adjointAccCopies copies
         end_ = acc + adjointAccCopies(ntype) * ntype * ntype;
@@ -70,7 +76,7 @@ __device__ __forceinline__ void adjointPairI(const IAtoms& I, const IGrad& Gi, c
     const float dx       = I.x[kI] - J.x;
     const float dy       = I.y[kI] - J.y;
     const float dz       = I.z[kI] - J.z;
-    float       rsq      = dx * dx + dy * dy + dz * dz;
+    float       rsq      = fmaf(dz, dz, fmaf(dx, dx, dy * dy)); // rounded as in the pair kernel
     float       interact = 1.0f;
     bool        skip;
     if (kChecks)
@@ -87,7 +93,6 @@ __device__ __forceinline__ void adjointPairI(const IAtoms& I, const IGrad& Gi, c
     // kernel)
     float rinv    = __builtin_amdgcn_rsqf(rsq);
     rinv          = skip ? 0.0f : rinv;
-    const float smask  = skip ? 0.0f : 1.0f;
     const float rinvsq = rinv * rinv;
     const float rinv3  = rinv * rinvsq;
 
@@ -105,7 +110,7 @@ __device__ __forceinline__ void adjointPairI(const IAtoms& I, const IGrad& Gi, c
     float hC, dhC;
     if (kElec == kElecRF)
     {
-        hC  = smask * (interact * rinv3 - 2.0f * ic.k_rf);
+        hC  = interact * rinv3 - (skip ? 0.0f : 2.0f * ic.k_rf);
         dhC = -1.5f * interact * rinv3 * rinvsq;
     }
     else if (kElec == kElecEwaldTable)
@@ -132,8 +137,10 @@ __device__ __forceinline__ void adjointPairI(const IAtoms& I, const IGrad& Gi, c
         const float rq  = __builtin_amdgcn_rcpf(qg);
         const float G   = pg * rq;
         const float dG  = (dpg - G * dqg) * rq;
-        hC              = smask * (interact * rinv3 - ic.beta3 * G);
-        dhC             = smask * (-1.5f * interact * rinv3 * rinvsq - ic.beta3 * ic.beta2 * dG);
+        // beyond the cut-off 1/r = 0 and the correction takes 0
+        const float b3 = skip ? 0.0f : ic.beta3;
+        hC             = interact * rinv3 - b3 * G;
+        dhC            = -1.5f * interact * rinv3 * rinvsq - b3 * ic.beta2 * dG;
     }
     const float qq  = I.q[kI] * J.w; // epsfac q_i q_j
     const float s   = fmaf(qq, hC, sLJ);
@@ -173,13 +180,10 @@ __device__ __forceinline__ void adjointTile(const IAtoms& I, const IGrad& Gi, co
 {
     adjointPairI<kElec, kParams, kChecks, 0>(I, Gi, J, gj, mbits, diag, jj, ic, sNbfp, sTab, sAcc, accStride,
                                              accCopies, ai, aj);
-    __builtin_amdgcn_sched_barrier(0);
     adjointPairI<kElec, kParams, kChecks, 1>(I, Gi, J, gj, mbits, diag, jj, ic, sNbfp, sTab, sAcc, accStride,
                                              accCopies, ai, aj);
-    __builtin_amdgcn_sched_barrier(0);
     adjointPairI<kElec, kParams, kChecks, 2>(I, Gi, J, gj, mbits, diag, jj, ic, sNbfp, sTab, sAcc, accStride,
                                              accCopies, ai, aj);
-    __builtin_amdgcn_sched_barrier(0);
     adjointPairI<kElec, kParams, kChecks, 3>(I, Gi, J, gj, mbits, diag, jj, ic, sNbfp, sTab, sAcc, accStride,
                                              accCopies, ai, aj);
 }
@@ -218,10 +222,7 @@ __global__ __launch_bounds__(kAdjThreads) void adjointKernel(const AdjointArgs a
     const int kk   = lane >> 2;
 
     const InteractionConst ic = a.ic;
-    float4* ix  = smem4 + L.ix + wave * kGroupSizeMax * kClusterSize;
-    float4* ig  = smem4 + L.ig + wave * kGroupSizeMax * kClusterSize;
-    int*    it  = reinterpret_cast<int*>(smem4 + L.it) + wave * kGroupSizeMax * kClusterSize;
-    float*  win = reinterpret_cast<float*>(smem4 + L.win) + wave * a.windowSlots * 16;
+    float* win = reinterpret_cast<float*>(smem4 + L.win) + wave * a.windowSlots * 16;
 
     // the wavefront's run of chunks, as in the forward kernel (the same
     // static schedule: wavefront w of the forward launch is wavefront w here)
@@ -236,11 +237,12 @@ __global__ __launch_bounds__(kAdjThreads) void adjointKernel(const AdjointArgs a
         const unsigned W0     = static_cast<unsigned>(uniformInt(cFirst.z));
         const int      T      = (uniformInt(cLast.z) - static_cast<int>(W0)) / kTileJ + uniformInt(cLast.w);
 
-        int    g = uniformInt(ws.y), chGrpEnd = 0, U = 0, c0 = 0, nOwn = 0, G = 0, stage = -1;
+        int    g = uniformInt(ws.y), chGrpEnd = 0, U = 0, c0 = 0, G = 0, stage = -1;
         IAtoms I;
         IGrad  Gi;
         float4 sv;
         float  ai[16];
+        unsigned spare = 0; // the slot after the window's last one
         int    ci = 0, sh = 0, nspec = 0, chStart = 0, chEnd = 0, chIdx = chAll0;
         bool   central = false;
 
@@ -250,19 +252,13 @@ __global__ __launch_bounds__(kAdjThreads) void adjointKernel(const AdjointArgs a
             const int4 si  = a.segInfo[gg];
             chGrpEnd       = uniformInt(grp.y);
             U              = uniformInt(grp.w);
+            spare = static_cast<unsigned>(uniformInt(gi.y) >> 16) + static_cast<unsigned>(U);
             stage = uniformInt(si.z) > 0 ? uniformInt(si.x) + (wid - uniformInt(si.y)) * uniformInt(si.w) : -1;
             c0             = uniformInt(gi.x);
-            nOwn           = uniformInt(gi.y) & 0xffff;
             G              = uniformInt(gi.y) >> 16;
             for (int t = lane; t < (G + U + 1) * 4; t += kWave)
             {
                 reinterpret_cast<float4*>(win)[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            }
-            if (lane < nOwn * kClusterSize)
-            {
-                ix[lane] = a.xq[c0 * kClusterSize + lane];
-                ig[lane] = a.gq[c0 * kClusterSize + lane];
-                it[lane] = a.type[c0 * kClusterSize + lane] * ntype;
             }
         };
         auto endGroup = [&]() {
@@ -285,21 +281,21 @@ __global__ __launch_bounds__(kAdjThreads) void adjointKernel(const AdjointArgs a
             central         = (sh == kCentral);
             chStart         = t;
             chEnd           = t + uniformInt(cd.w);
-            const int lc    = (ci - c0) * kClusterSize;
+            const Float16 p  = scalarLoad<Float16>(a.xq + ci * kClusterSize);
+            const Float16 q  = scalarLoad<Float16>(a.gq + ci * kClusterSize);
+            const Int4    ty = scalarLoad<Int4>(a.type + ci * kClusterSize);
 #pragma unroll
             for (int i = 0; i < 4; i++)
             {
-                const float4 p = ix[lc + i];
-                I.x[i]         = uniformFloat(p.x);
-                I.y[i]         = uniformFloat(p.y);
-                I.z[i]         = uniformFloat(p.z);
-                I.q[i]         = uniformFloat(p.w);
-                I.tOff[i]      = uniformInt(it[lc + i]);
-                const float4 q = ig[lc + i];
-                Gi.x[i]        = uniformFloat(q.x);
-                Gi.y[i]        = uniformFloat(q.y);
-                Gi.z[i]        = uniformFloat(q.z);
-                Gi.qe[i]       = uniformFloat(p.w * ic.epsfac);
+                I.x[i]    = p[4 * i];
+                I.y[i]    = p[4 * i + 1];
+                I.z[i]    = p[4 * i + 2];
+                I.q[i]    = p[4 * i + 3];
+                I.tOff[i] = ty[i] * ntype;
+                Gi.x[i]   = q[4 * i];
+                Gi.y[i]   = q[4 * i + 1];
+                Gi.z[i]   = q[4 * i + 2];
+                Gi.qe[i]  = q[4 * i + 3];
             }
             sv = make_float4(uniformFloat(sf.x), uniformFloat(sf.y), uniformFloat(sf.z), 0.0f);
 #pragma unroll
@@ -316,8 +312,15 @@ __global__ __launch_bounds__(kAdjThreads) void adjointKernel(const AdjointArgs a
             }
         };
         auto doTile = [&](const uint2 e, const float4 xj, const int tj, const float4 gj, const bool checked) {
-            const JAtom J{ xj.x - sv.x, xj.y - sv.y, xj.z - sv.z, ic.epsfac * xj.w, tj };
+            // gq's w holds epsfac q
+            const JAtom J{ xj.x - sv.x, xj.y - sv.y, xj.z - sv.z, gj.w, tj };
             float4      aj = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            // the window's sums are read before the pair arithmetic, which
+            // covers the read's latency; lanes whose cluster did not fit the
+            // window use the spare slot, as padding entries do
+            const unsigned slot = e.y >> 16;
+            float4* const  w    = reinterpret_cast<float4*>(win + min(slot, spare) * 16 + jj * 4);
+            float4         v    = *w;
             if (checked)
             {
                 const bool diag = central && static_cast<int>(e.x) == ci;
@@ -329,18 +332,12 @@ __global__ __launch_bounds__(kAdjThreads) void adjointKernel(const AdjointArgs a
                 adjointTile<kElec, kParams, false>(I, Gi, J, gj, 0u, false, jj, ic, sNbfp, sTab, sAcc, accStride,
                                                    accCopies, ai, aj);
             }
-            const unsigned slot = e.y >> 16;
-            if (slot != kSlotOverflow)
-            {
-                float4* w = reinterpret_cast<float4*>(win + slot * 16 + jj * 4);
-                float4  v = *w;
-                v.x += aj.x;
-                v.y += aj.y;
-                v.z += aj.z;
-                v.w += aj.w;
-                *w = v;
-            }
-            else
+            v.x += aj.x;
+            v.y += aj.y;
+            v.z += aj.z;
+            v.w += aj.w;
+            *w = v;
+            if (slot == kSlotOverflow)
             {
                 const int k   = static_cast<int>(e.x) * kClusterSize + jj;
                 float*    dst = reinterpret_cast<float*>(a.gradX + k);
@@ -366,16 +363,23 @@ __global__ __launch_bounds__(kAdjThreads) void adjointKernel(const AdjointArgs a
             svNext = a.chunkShift[min(chIdx + 1, chAll1 - 1)];
         };
 
-        // the forward kernel's pipeline: work entries two tiles ahead, j-atom
-        // data one tile ahead; reads past the last tile are clamped to it
+        // the forward kernel's pipeline: work entries four tiles ahead, j-atom
+        // data two tiles ahead; reads past the last tile are clamped to it
         auto entryAt = [&](int t) {
             return ldg(a.work, W0 + static_cast<unsigned>(kTileJ * min(t, T - 1) + kk));
         };
-        uint2  eA = entryAt(0);
-        uint2  eB = entryAt(1);
-        float4 xA = ldg(a.xq, eA.x * kClusterSize + jj);
-        int    tA = ldg(a.type, eA.x * kClusterSize + jj);
-        float4 gA = ldg(a.gq, eA.x * kClusterSize + jj);
+        struct Atoms
+        {
+            float4 x, g;
+            int    type;
+        };
+        auto load = [&](const uint2 e) {
+            const unsigned k = e.x * kClusterSize + jj;
+            return Atoms{ ldg(a.xq, k), ldg(a.gq, k), ldg(a.type, k) };
+        };
+        // tiles t and t + 1 (entries, j-atoms), entries of t + 2 and t + 3
+        uint2 e0 = entryAt(0), e1 = entryAt(1), e2 = entryAt(2), e3 = entryAt(3);
+        Atoms x0 = load(e0), x1 = load(e1);
         beginGroup(g);
         beginChunk(cFirst, a.chunkShift[chAll0], 0);
         // an odd tile count: the first tile alone, so that the loop below
@@ -388,36 +392,41 @@ __global__ __launch_bounds__(kAdjThreads) void adjointKernel(const AdjointArgs a
             {
                 advance(0);
             }
-            doTile(eA, xA, tA, gA, 0 - chStart < nspec);
-            xA = ldg(a.xq, eB.x * kClusterSize + jj);
-            tA = ldg(a.type, eB.x * kClusterSize + jj);
-            gA = ldg(a.gq, eB.x * kClusterSize + jj);
-            eA = eB;
-            eB = entryAt(2);
+            doTile(e0, x0.x, x0.type, x0.g, 0 - chStart < nspec);
+            e0 = e1;
+            e1 = e2;
+            e2 = e3;
+            e3 = entryAt(4);
+            x0 = x1;
+            x1 = load(e1);
             t0 = 1;
         }
         for (int t = t0; t < T; t += 2)
         {
-            const float4 xB  = ldg(a.xq, eB.x * kClusterSize + jj);
-            const int    tB  = ldg(a.type, eB.x * kClusterSize + jj);
-            const float4 gB  = ldg(a.gq, eB.x * kClusterSize + jj);
-            const uint2  eA2 = entryAt(t + 2);
             if (t == chEnd)
             {
                 advance(t);
             }
-            doTile(eA, xA, tA, gA, t - chStart < nspec);
-            const uint2 eB2 = entryAt(t + 3);
-            xA              = ldg(a.xq, eA2.x * kClusterSize + jj);
-            tA              = ldg(a.type, eA2.x * kClusterSize + jj);
-            gA              = ldg(a.gq, eA2.x * kClusterSize + jj);
+            {
+                const Atoms x  = x0;
+                const uint2 e4 = entryAt(t + 4);
+                x0             = load(e2);
+                doTile(e0, x.x, x.type, x.g, t - chStart < nspec);
+                e0 = e2;
+                e2 = e4;
+            }
             if (t + 1 == chEnd)
             {
                 advance(t + 1);
             }
-            doTile(eB, xB, tB, gB, t + 1 - chStart < nspec);
-            eA = eA2;
-            eB = eB2;
+            {
+                const Atoms x  = x1;
+                const uint2 e5 = entryAt(t + 5);
+                x1             = load(e3);
+                doTile(e1, x.x, x.type, x.g, t + 1 - chStart < nspec);
+                e1 = e3;
+                e3 = e5;
+            }
         }
         endChunk();
         endGroup();
@@ -605,7 +614,8 @@ __global__ __launch_bounds__(256) void adjointFinishKernel(int paramBlocks, int 
 }
 
 __global__ void adjointPrepareKernel(int nslot, const int* __restrict__ atomIndices, const float* __restrict__ x,
-                                     const float* __restrict__ g, float4* __restrict__ xq, float4* __restrict__ gq,
+                                     const float* __restrict__ g, float epsfac, float4* __restrict__ xq,
+                                     float4* __restrict__ gq,
                                      float4* __restrict__ gradX, double* __restrict__ gradQ)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -622,7 +632,9 @@ __global__ void adjointPrepareKernel(int nslot, const int* __restrict__ atomIndi
         v.z      = x[3 * a + 2];
         xq[s]    = v;
     }
-    gq[s] = a >= 0 ? make_float4(g[3 * a + 0], g[3 * a + 1], g[3 * a + 2], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    // w: epsfac q, which the kernel needs of both atoms of a pair
+    gq[s] = a >= 0 ? make_float4(g[3 * a + 0], g[3 * a + 1], g[3 * a + 2], epsfac * xq[s].w)
+                   : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (s < nslot)
     {
         gradX[s] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -695,11 +707,11 @@ void launchAdjoint(hipStream_t s, const AdjointArgs& a, int elec, int forwardBlo
     }
 }
 
-void launchAdjointPrepare(hipStream_t s, int nslot, const int* atomIndices, const float* x, const float* g, float4* xq,
-                          float4* gq, float4* gradX, double* gradQ)
+void launchAdjointPrepare(hipStream_t s, int nslot, const int* atomIndices, const float* x, const float* g,
+                          float epsfac, float4* xq, float4* gq, float4* gradX, double* gradQ)
 {
-    adjointPrepareKernel<<<(nslot + kClusterSize + 255) / 256, 256, 0, s>>>(nslot, atomIndices, x, g, xq, gq, gradX,
-                                                                           gradQ);
+    adjointPrepareKernel<<<(nslot + kClusterSize + 255) / 256, 256, 0, s>>>(nslot, atomIndices, x, g, epsfac, xq, gq,
+                                                                           gradX, gradQ);
 }
 
 } // namespace nbx

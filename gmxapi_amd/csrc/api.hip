@@ -324,10 +324,9 @@ int stagedGroupSize(const nbx_context* c, bool adjoint)
 {
     const double nc = std::max(c->ncluster, 1);
     const double nj = static_cast<double>(c->ncj) / nc;
-    // the wavefronts of the launch: two per SIMD for the pair kernel (three
-    // two-wavefront workgroups per CU for the adjoint), or this system's
-    // share of a batch's launch
-    const double resident = c->numCU * (adjoint ? 6.0 : 2.0 * kKernelWaves);
+    // the wavefronts of the launch: two per SIMD, or this system's share of a
+    // batch's launch
+    const double resident = c->numCU * 2.0 * (adjoint ? kAdjointWaves : kKernelWaves);
     const double waves    = !adjoint && c->batchWaves > 0 ? c->batchWaves : std::min(resident, std::max(1.0, 1.0 * c->nci));
     double       least    = 0.0;
     int          best     = 1;
@@ -402,7 +401,7 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
         {
             si++;
         }
-        const int  budget   = adjoint ? adjointLayoutBudget(c->ntype) : kKernelLdsBudget;
+        const int  budget   = adjoint ? kAdjointLayoutBudget : kKernelLdsBudget;
         if (!fallback && forced > 0 && G != forced)
         {
             continue;
@@ -537,17 +536,16 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
 // The layout's grid and static schedule (the workgroups that can be
 // resident, every wavefront a contiguous run of chunks of about equal cost)
 // and its window staging.  The pair kernel runs kKernelWaves wavefronts per
-// workgroup; the adjoint two (its numBlocks counts groups of four
-// wavefronts, as the schedule does).
+// workgroup, the adjoint kAdjointWaves.
 void scheduleLayout(nbx_context* c, WorkLayout& L, bool adjoint)
 {
     int numWaves;
     if (adjoint)
     {
         const int lds   = adjointLdsBytes(c->ntype, c->ic.tab_n, c->elec, L.windowSlots);
-        const int perCU = std::max(1, std::min(8, (160 * 1024) / lds)); // two-wavefront workgroups
+        const int perCU = std::max(1, std::min(2, (160 * 1024) / lds));
         numWaves        = std::max(kKernelWaves, std::min((L.nchunk + kKernelWaves - 1) / kKernelWaves * kKernelWaves,
-                                                          perCU * c->numCU * 2));
+                                                          perCU * c->numCU * kAdjointWaves));
         numWaves        = (numWaves + kKernelWaves - 1) / kKernelWaves * kKernelWaves;
     }
     else
@@ -576,7 +574,8 @@ void scheduleLayout(nbx_context* c, WorkLayout& L, bool adjoint)
     else
     {
         launchWaveSchedule(c->stream, numWaves, L.nchunk, L.chunks.p, L.nwork,
-                           adjoint ? kAdjointChunkWeight : kChunkWeight, L.ngroups, L.groups.p, L.waveStart.p);
+                           adjoint ? kAdjointChunkWeight : kChunkWeight, L.ngroups, L.groups.p, L.waveStart.p, nullptr,
+                           nullptr, c->numCU * (adjoint ? kAdjointWaves : kKernelWaves));
     }
     check(hipGetLastError(), "schedule kernel");
     buildSegments(c->stream, L.gather, L.ngroups, L.groups.p, L.groupInfo.p, numWaves, L.waveStart.p, c->ncluster,
@@ -1788,7 +1787,8 @@ int nbx_compute_adjoint(nbx_context* c, const float* x, const float* g, float* g
         c->gq.ensure(nslot + kClusterSize);
         c->gradXnb.ensure(nslot + kClusterSize);
         c->gradQnb.ensure(nslot + kClusterSize);
-        launchAdjointPrepare(c->stream, nslot, c->atomIndices.p, xd, gd, c->xq.p, c->gq.p, c->gradXnb.p, c->gradQnb.p);
+        launchAdjointPrepare(c->stream, nslot, c->atomIndices.p, xd, gd, c->ic.epsfac, c->xq.p, c->gq.p, c->gradXnb.p,
+                             c->gradQnb.p);
         const int    blocks = adjointBlocks(c->adj.numBlocks);
         const size_t np     = 2 * static_cast<size_t>(c->ntype) * c->ntype;
         c->paramPartial.ensure(blocks * np);

@@ -78,22 +78,18 @@ constexpr int kGenerationSkewMilli = 80;
 constexpr int kKernelWaves      = 4;
 constexpr int kKernelLdsBudget  = 80 * 1024;
 constexpr int kAdjointLdsBudget = 160 * 1024;
-// LDS per two-wavefront adjoint workgroup that its group size is chosen for
-// (three resident workgroups per CU)
-constexpr int kAdjointLayoutBudget = 48 * 1024;
+// wavefronts per adjoint workgroup, and the LDS that its group size is chosen
+// for (two resident workgroups per CU)
+constexpr int kAdjointWaves        = 4;
+constexpr int kAdjointLayoutBudget = 80 * 1024;
 // copies of the adjoint's per-workgroup C6/C12 accumulators in LDS (lanes
-// spread over them, fewer lanes per address in each LDS atomic); the layout
-// budget grows by the copies beyond the first
+// spread over them, fewer lanes per address in each LDS atomic)
 #ifndef NBX_ADJ_ACC_COPIES
 #define NBX_ADJ_ACC_COPIES 2
 #endif
 __host__ __device__ inline int adjointAccCopies(int ntype)
 {
     return ntype <= 24 ? NBX_ADJ_ACC_COPIES : 1;
-}
-__host__ __device__ inline int adjointLayoutBudget(int ntype)
-{
-    return kAdjointLayoutBudget + (adjointAccCopies(ntype) - 1) * ntype * ntype * 16;
 }
 // rsq floor for float (pairlist.h:146): r > 6.2e-4 nm; and a cap far beyond
 // any cut-off that keeps products of the masked 1/r = 0 finite
@@ -500,7 +496,7 @@ struct AdjointArgs
     const int*    unionList;
     const uint2*  work;
     const float4* xq;
-    const float4* gq; // dL/dF per cluster-layout atom (w unused)
+    const float4* gq; // per cluster-layout atom: dL/dF and, in w, epsfac q
     const int*    type;
     const float2* nbfp;
     int           ntype;
@@ -529,8 +525,8 @@ void launchAdjoint(hipStream_t s, const AdjointArgs& a, int elec, int forwardBlo
                    float* gradXOut, double* gradQOut, int numTypes, double* gradC6Out, double* gradC12Out);
 // coordinates (x may be NULL) and g into the cluster layout, spill
 // accumulators cleared: xq, gq hold nslot + 4 entries (the padding cluster)
-void launchAdjointPrepare(hipStream_t s, int nslot, const int* atomIndices, const float* x, const float* g, float4* xq,
-                          float4* gq, float4* gradX, double* gradQ);
+void launchAdjointPrepare(hipStream_t s, int nslot, const int* atomIndices, const float* x, const float* g,
+                          float epsfac, float4* xq, float4* gq, float4* gradX, double* gradQ);
 
 // -- buffers.hip
 // zeroes n float4 and, when d is not NULL, nd doubles

@@ -98,3 +98,25 @@ def test_results_follow_the_last_step():
     ctx.compute(s.x)
     with pytest.raises(nbx.NbxStateError):
         ctx.energies()
+
+
+@pytest.mark.parametrize("natoms,ntypes,correction,bar", [
+    (1500, 31, "table", 2e-3),       # the most types: the smallest windows, which overflow
+    (1500, 24, "analytical", 1e-4),  # one copy of the C6/C12 accumulators
+    (1010, 1, "analytical", 1e-4),   # fewer tiles than wavefronts
+])
+def test_adjoint_at_the_limits_of_its_lds(natoms, ntypes, correction, bar):
+    # the adjoint's bars (test_gpu_adjoint.py) where its LDS is shared out
+    # differently: FP32 pair terms against the FP64 reference gradient
+    from oracle import adjoint as A
+
+    print(f"[adjoint] {natoms} atoms, {ntypes} types, {correction}", flush=True)
+    s = S.hetero_chains(natoms, max(2.51, (natoms / 100.0) ** (1 / 3)), ntypes=ntypes, seed=ntypes)
+    g = np.random.default_rng(2).normal(size=s.x.shape)
+    ref = A.forces_and_gradient(s, g, s.c6_matrix(), s.c12_matrix(), pairs=A.pair_table(s.x, s.box, s.rcoulomb))
+    gx, gq, g6, g12 = nbx.context_for(s, ewald_correction=correction).compute_adjoint(s.x, g)
+    assert rms(gx - ref["grad_x"]) <= bar * rms(ref["grad_x"])
+    assert rms((gq - ref["grad_q"])[:, None]) <= bar * rms(ref["grad_q"][:, None])
+    for got, want in ((g6, ref["grad_c6"]), (g12, ref["grad_c12"])):
+        got, want = A.symmetrized(got), A.symmetrized(want)
+        assert np.abs(got - want).max() <= bar * np.abs(want).max()
