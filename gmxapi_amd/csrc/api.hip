@@ -311,6 +311,13 @@ static void ensureStats(nbx_context* c)
     c->statsPartial.ensure(kStatsHead + kPartialMaxBlocks * partialMaxStride(2, true));
 }
 
+// the forward kernel's schedule by the measured cost model (unless the cost
+// total could overflow an int)
+bool useCostModel(const nbx_context* c, bool adjoint)
+{
+    return !adjoint && scheduleCostBound(c->numWork, c->nci, kCostChunk) < INT_MAX;
+}
+
 // The group size beyond which larger groups stage more.  Every (wavefront,
 // group) pair clears, stages and gathers one window, and every wavefront but
 // the first starts inside some group, so (nc / G + waves) windows of U(G) + G
@@ -346,7 +353,9 @@ int stagedGroupSize(const nbx_context* c, bool adjoint)
 // (groups.hip): the largest group size whose j-entries fit the LDS sort and
 // whose window fits the kernel's LDS budget (the pair kernel's, or with
 // adjoint the adjoint kernel's, whose window holds 4 floats per atom).
-void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spansKnown = nullptr)
+// searchCap > 0: the list is still where the search left it (regions of
+// searchCap j-entries per cluster); the pass makes it compact.
+void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spansKnown = nullptr, int searchCap = 0)
 {
     auto ldsBytes = [&](int slots) {
         return adjoint ? adjointLdsBytes(c->ntype, c->ic.tab_n, c->elec, slots)
@@ -370,7 +379,10 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
         check(hipStreamSynchronize(c->stream), "group sync");
         reducePartialMax(hp, nb, kGroupSizeCount, spans);
     }
-    c->jentryTmp.ensure(c->ncj);
+    if (searchCap == 0)
+    {
+        c->jentryTmp.ensure(c->ncj);
+    }
     // the largest group size up to stagedGroupSize (or the chosen one) whose
     // j-force windows, one per wavefront, fit the workgroup's LDS budget:
     // larger groups share more j-clusters per flush, which pays more than a
@@ -415,118 +427,112 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
             throw InputError("a grid cluster has more than " + std::to_string(kGroupMaxJ)
                              + " cluster-pair entries: the pair-list cut-off is too long for this kernel");
         }
-        const int ng = (nc + G - 1) / G;
+        // the most window slots the budget holds
+        int cap = G + kGroupMaxJ + 1;
+        if (ldsBytes(cap) > budget)
+        {
+            int fits = G + 1, over = cap;
+            while (over - fits > 1)
+            {
+                const int mid = (fits + over) / 2;
+                (ldsBytes(mid) <= budget ? fits : over) = mid;
+            }
+            cap = fits;
+            if (cap < G + 2)
+            {
+                continue;
+            }
+        }
+        const int  ng        = (nc + G - 1) / G;
+        const bool costModel = useCostModel(c, adjoint);
         L.unionCount.ensure(ng + 1);
-        L.chunkCount.ensure(ng + 1);
-        L.workCount.ensure(ng + 1);
-        L.overflow.ensure(ng + 1);
+        L.spillCount.ensure(ng + 1);
         L.unionOff.ensure(scanOutSize(ng));
-        L.chunkOff.ensure(scanOutSize(ng));
-        L.workOff.ensure(scanOutSize(ng));
+        L.spillOff.ensure(scanOutSize(ng));
         L.groups.ensure(ng);
         L.groupInfo.ensure(ng);
-        // one pass writes the layout at upper-bound bases (no count pass);
-        // the scans of its per-group counts give the compact offsets
         L.unionTmp.ensure(std::max(c->ncj, 1));
-        L.chunksTmp.ensure(std::max(c->nci, 1));
-        L.workTmp.ensure(std::max(c->ncj + (kTileJ - 1) * c->nci, 1));
+        L.chunks.ensure(std::max(c->nci, 1));
+        L.chunkShift.ensure(std::max(c->nci, 1));
+        L.work.ensure(std::max(c->numWork, 1));
+        L.gather.occCount.ensure(nc + 1);
+        if (costModel)
+        {
+            L.chunkCost.ensure(c->nci + 2);
+        }
         GroupArgs ga{};
-        ga.ncluster     = nc;
-        ga.groupSize    = G;
-        ga.ngroups      = ng;
-        ga.chunkEntries = kChunkEntries;
-        ga.offI         = c->offI.p;
-        ga.offJ         = c->offJ.p;
-        ga.ientry       = c->ientry.p;
-        ga.jentryIn     = c->jentry.p;
-        ga.jentryOut    = c->jentryTmp.p;
-        ga.unionCount   = L.unionCount.p;
-        ga.chunkCount   = L.chunkCount.p;
-        ga.workCount    = L.workCount.p;
-        ga.overflow     = L.overflow.p;
-        ga.unionOff     = L.unionOff.p;
-        ga.chunkOff     = L.chunkOff.p;
-        ga.workOff      = L.workOff.p;
-        ga.unionList    = L.unionTmp.p;
-        ga.work         = L.workTmp.p;
-        ga.chunks       = L.chunksTmp.p;
-        ga.groups       = L.groups.p;
-        ga.groupInfo    = L.groupInfo.p;
-        ga.windowCap    = 1 << 30; // uncapped slots; the compaction applies the window capacity
-        ga.upperBound   = 1;
-        ga.unionBySort  = unionBySort ? 1 : 0;
-        launchBuildGroups(c->stream, ga, true);
-        // the largest union and the overflow flag, as per-workgroup maxima
-        // after the three scan totals (one read)
+        ga.ncluster    = nc;
+        ga.groupSize   = G;
+        ga.ngroups     = ng;
+        ga.offI        = c->offI.p;
+        ga.offJ        = c->offJ.p;
+        ga.offW        = c->offW.p;
+        ga.capJ        = searchCap;
+        ga.ientryIn    = searchCap > 0 ? c->searchITmp.p : c->ientry.p;
+        ga.jentryIn    = searchCap > 0 ? c->searchJTmp.p : c->jentry.p;
+        ga.ientryOut   = c->ientry.p;
+        ga.jentryOut   = searchCap > 0 ? c->jentry.p : c->jentryTmp.p;
+        ga.unionCount  = L.unionCount.p;
+        ga.spillCount  = L.spillCount.p;
+        ga.unionTmp    = L.unionTmp.p;
+        ga.work        = L.work.p;
+        ga.chunks      = L.chunks.p;
+        ga.chunkShift  = L.chunkShift.p;
+        ga.shiftVec    = c->shiftVec.p;
+        ga.chunkCost   = costModel ? L.chunkCost.p : nullptr;
+        ga.type        = c->nbtype.p;
+        ga.typeLJ      = c->typeLJ.p;
+        ga.windowCap   = cap;
+        ga.unionBySort = unionBySort ? 1 : 0;
+        ga.unionOff    = L.unionOff.p;
+        ga.groups      = L.groups.p;
+        ga.groupInfo   = L.groupInfo.p;
+        ga.occCount    = L.gather.occCount.p;
+        launchBuildGroups(c->stream, ga);
+        // the largest union, as per-workgroup maxima after the totals of the
+        // unions and of what lies beyond the windows (one read)
         ensureStats(c);
-        const PartialMaxArgs pm{ { L.unionCount.p, L.overflow.p }, 2, nullptr, ng, c->statsPartial.p + kStatsHead };
+        const PartialMaxArgs pm{ { L.unionCount.p, nullptr }, 1, nullptr, ng, c->statsPartial.p + kStatsHead };
         const int            statBlocks = launchPartialMax(c->stream, pm);
         {
-            const int* in[3]  = { L.unionCount.p, L.chunkCount.p, L.workCount.p };
-            int*       out[3] = { L.unionOff.p, L.chunkOff.p, L.workOff.p };
-            int*       tot[3] = { c->statsPartial.p, c->statsPartial.p + 1, c->statsPartial.p + 2 };
-            launchExclusiveScansWide(c->stream, ng, 3, in, out, tot);
+            const int* in[2]  = { L.unionCount.p, L.spillCount.p };
+            int*       out[2] = { L.unionOff.p, L.spillOff.p };
+            int*       tot[2] = { c->statsPartial.p, c->statsPartial.p + 1 };
+            launchExclusiveScansWide(c->stream, ng, 2, in, out, tot);
         }
         int* const hp = pinnedInts();
-        check(hipMemcpyAsync(hp, c->statsPartial.p, sizeof(int) * (kStatsHead + statBlocks * 2), hipMemcpyDeviceToHost,
+        check(hipMemcpyAsync(hp, c->statsPartial.p, sizeof(int) * (kStatsHead + statBlocks), hipMemcpyDeviceToHost,
                              c->stream),
               "read stats");
         check(hipStreamSynchronize(c->stream), "group sync");
-        int mx[2];
-        reducePartialMax(hp + kStatsHead, statBlocks, 2, mx);
-        const int maxUnion = mx[0], overflow = mx[1], unionTotal = hp[0], chunkTotal = hp[1], workTotal = hp[2];
-        if (overflow)
-        {
-            continue;
-        }
-        // window capacity: own clusters, the union, and the padding entries'
+        int maxUnion = 0;
+        reducePartialMax(hp + kStatsHead, statBlocks, 1, &maxUnion);
+        const int       unionTotal = hp[0];
+        const long long spilled    = hp[1];
+        // window slots: own clusters, the union, and the padding entries'
         // spare slot; when the largest union does not fit the budget, the
         // window holds the first union clusters of each group and the rest
         // take direct global atomics, which is accepted while that is at most
         // 2% of the union entries (any share in the last pass)
-        int slots = G + maxUnion + 1;
-        L.spill   = false;
-        if (ldsBytes(slots) > budget)
+        if (!fallback && spilled * 50 > unionTotal)
         {
-            while (slots > G + 2 && ldsBytes(slots) > budget)
-            {
-                slots--;
-            }
-            if (ldsBytes(slots) > budget)
-            {
-                continue;
-            }
-            std::vector<int> counts(ng);
-            check(hipMemcpy(counts.data(), L.unionCount.p, sizeof(int) * ng, hipMemcpyDeviceToHost), "read unions");
-            long long spilled = 0;
-            for (int u : counts)
-            {
-                spilled += std::max(0, u - (slots - 1 - G));
-            }
-            if (!fallback && spilled * 50 > unionTotal)
-            {
-                continue;
-            }
-            L.spill = spilled > 0;
+            continue;
         }
-        // the compaction gives union clusters beyond the window the overflow slot
-        ga.windowCap = slots;
+        const int slots = std::min(G + maxUnion + 1, cap);
+        L.spill         = spilled > 0;
         L.unionList.ensure(std::max(unionTotal, 1));
-        L.chunks.ensure(std::max(chunkTotal, 1));
-        L.work.ensure(std::max(workTotal, 1));
         ga.unionList = L.unionList.p;
-        ga.work      = L.work.p;
-        ga.chunks    = L.chunks.p;
-        launchGroupCompact(c->stream, ga, L.unionTmp.p, L.workTmp.p, L.chunksTmp.p);
-        L.chunkShift.ensure(std::max(chunkTotal, 1));
-        launchChunkShifts(c->stream, chunkTotal, L.chunks.p, c->shiftVec.p, L.chunkShift.p);
+        launchGroupUnions(c->stream, ga);
         check(hipGetLastError(), "group kernels");
-        c->jentry.swap(c->jentryTmp);
-        buildOccurrences(c->stream, L.gather, ng, L.groups.p, L.groupInfo.p, L.unionList.p, nc, nc + unionTotal);
+        if (searchCap == 0)
+        {
+            c->jentry.swap(c->jentryTmp);
+        }
+        buildOccurrences(c->stream, L.gather, ng, L.groups.p, L.groupInfo.p, L.unionList.p, nc, nc + unionTotal, true);
         L.groupSize   = G;
         L.ngroups     = ng;
-        L.nchunk      = chunkTotal;
-        L.nwork       = workTotal;
+        L.nchunk      = c->nci;
+        L.nwork       = c->numWork;
         L.windowSlots = slots;
         return;
     }
@@ -558,15 +564,11 @@ void scheduleLayout(nbx_context* c, WorkLayout& L, bool adjoint)
     }
     L.numBlocks = numWaves / kKernelWaves;
     L.waveStart.ensure(numWaves + 1);
-    // the forward kernel's runs by the measured cost model (unless the cost
-    // total could overflow an int), with the first of two resident
-    // generations of workgroups taking the larger share
-    if (!adjoint && scheduleCostBound(L.nwork, L.nchunk, kCostChunk) < INT_MAX)
+    // the first of two resident generations of workgroups takes the larger
+    // share
+    if (useCostModel(c, adjoint))
     {
-        L.chunkCost.ensure(L.nchunk + 2);
         L.costOff.ensure(scanOutSize(L.nchunk));
-        launchChunkCosts(c->stream, L.nchunk, L.chunks.p, c->nbtype.p, c->typeLJ.p, kCostChunk,
-                         L.chunkCost.p);
         launchExclusiveScanWide(c->stream, L.nchunk, L.chunkCost.p, L.costOff.p, L.chunkCost.p + L.nchunk + 1);
         launchWaveSchedule(c->stream, numWaves, L.nchunk, L.chunks.p, L.nwork, kChunkWeight, L.ngroups, L.groups.p,
                            L.waveStart.p, L.costOff.p, L.chunkCost.p + L.nchunk + 1, c->numCU * kKernelWaves);
@@ -1219,9 +1221,9 @@ int nbx_put_on_grid(nbx_context* c, const float* box, const float* x, int xOnDev
 
 // After a search or a prune: the pair kernel's work layout and schedule and
 // the per-step output buffers sized for it.
-static void finishList(nbx_context* c, const int* spans = nullptr)
+static void finishList(nbx_context* c, const int* spans = nullptr, int searchCap = 0)
 {
-    buildWorkGroups(c, c->lay, false, spans);
+    buildWorkGroups(c, c->lay, false, spans, searchCap);
     scheduleLayout(c, c->lay, false);
     const int numWaves = c->lay.numBlocks * kKernelWaves;
     c->energyPartial.ensure(2 * static_cast<size_t>(c->lay.ngroups + numWaves));
@@ -1247,8 +1249,10 @@ int nbx_construct_pairlist(nbx_context* c)
         const int nc = c->ncluster;
         c->countJ.ensure(nc + 1);
         c->countI.ensure(nc + 1);
+        c->countW.ensure(nc + 1);
         c->offJ.ensure(scanOutSize(nc));
         c->offI.ensure(scanOutSize(nc));
+        c->offW.ensure(scanOutSize(nc));
         c->totals.ensure(3);
         ensureStats(c);
         SearchArgs a{};
@@ -1265,14 +1269,15 @@ int nbx_construct_pairlist(nbx_context* c)
         a.exclIdx     = c->exclIdx.p;
         a.countJ      = c->countJ.p;
         a.countI      = c->countI.p;
+        a.countW      = c->countW.p;
         a.offJ        = c->offJ.p;
         a.offI        = c->offI.p;
-        // the j- and i-entry counts scanned together (two workgroups, one launch)
+        // the j-, i- and padded work entry counts scanned together
         auto scanCounts = [&] {
-            const int* in[2]  = { c->countJ.p, c->countI.p };
-            int*       out[2] = { c->offJ.p, c->offI.p };
-            int*       tot[2] = { c->statsPartial.p, c->statsPartial.p + 1 };
-            launchExclusiveScansWide(c->stream, nc, 2, in, out, tot);
+            const int* in[3]  = { c->countJ.p, c->countI.p, c->countW.p };
+            int*       out[3] = { c->offJ.p, c->offI.p, c->offW.p };
+            int*       tot[3] = { c->statsPartial.p, c->statsPartial.p + 1, c->statsPartial.p + 2 };
+            launchExclusiveScansWide(c->stream, nc, 3, in, out, tot);
         };
         // the list's totals, its largest j-entry count and the group pass's
         // largest j-entry span per group size (per-workgroup maxima), read
@@ -1293,16 +1298,18 @@ int nbx_construct_pairlist(nbx_context* c)
             const int* hp = pinnedInts();
             int        st[partialMaxStride(1, true)];
             reducePartialMax(hp + kStatsHead, statBlocks, partialMaxStride(1, true), st);
-            tot[0] = hp[0];
-            tot[1] = hp[1];
-            tot[2] = st[0];
+            tot[0]     = hp[0];
+            tot[1]     = hp[1];
+            tot[2]     = st[0];
+            c->numWork = hp[2];
             std::copy(st + 1, st + 1 + kGroupSizeCount, spans);
         };
         // After a first search, the fill runs without a count pass: each
         // cluster writes into a region sized from the largest count seen
-        // (with a margin) and a compaction follows the scans; a cluster that
+        // (with a margin) and the group pass makes it compact; a cluster that
         // outgrows it sends the search through the counted path again.
-        bool done = false;
+        bool done      = false;
+        int  searchCap = 0;
         if (c->searchCapJ > 0)
         {
             const int cap = c->searchCapJ;
@@ -1323,8 +1330,7 @@ int nbx_construct_pairlist(nbx_context* c)
                 c->nci = tot[1];
                 c->ientry.ensure(c->nci);
                 c->jentry.ensure(c->ncj);
-                launchSearchCompact(c->stream, nc, cap, c->countJ.p, c->countI.p, c->offJ.p, c->offI.p,
-                                    c->searchJTmp.p, c->searchITmp.p, c->jentry.p, c->ientry.p);
+                searchCap     = cap;
                 c->searchCapJ = tot[2] + tot[2] / 4 + 32;
                 done          = true;
             }
@@ -1352,7 +1358,7 @@ int nbx_construct_pairlist(nbx_context* c)
         check(hipGetLastError(), "search kernels");
         launchExclusionSlots(c->stream, c->numExclPairs, c->exclPairs.p, c->cells.p, c->exclPairSlots.p);
         c->haveOuter = false;
-        finishList(c, spans);
+        finishList(c, spans, searchCap);
     });
 }
 
@@ -1419,7 +1425,11 @@ int nbx_prune_pairlist(nbx_context* c, double rlistInner)
         a.ientry = c->ientry.p;
         a.jentry = c->jentry.p;
         launchPrune(c->stream, a, true);
+        launchClusterWork(c->stream, nc, c->offI.p, c->ientry.p, c->countW.p);
+        launchExclusiveScanWide(c->stream, nc, c->countW.p, c->offW.p, c->totals.p + 2);
         check(hipGetLastError(), "prune kernels");
+        check(hipMemcpyAsync(&c->numWork, c->totals.p + 2, sizeof(int), hipMemcpyDeviceToHost, c->stream), "read totals");
+        check(hipStreamSynchronize(c->stream), "prune sync");
         finishList(c);
     });
 }

@@ -149,8 +149,9 @@ struct WindowGather
 // A group lists its own clusters and its windowed union, so the lists hold
 // at most ncluster + (union entries of all groups) = maxTotal occurrences:
 // with maxTotal given the host does not wait for the exact count.
+// counted: launchGroupUnions has put the counts into w.occCount.
 inline void buildOccurrences(hipStream_t s, WindowGather& w, int ngroups, const int4* groups, const int4* groupInfo,
-                             const int* unionList, int ncluster, int maxTotal = -1)
+                             const int* unionList, int ncluster, int maxTotal, bool counted)
 {
     w.occCount.ensure(ncluster + 1);
     w.occOff.ensure(scanOutSize(ncluster));
@@ -160,19 +161,13 @@ inline void buildOccurrences(hipStream_t s, WindowGather& w, int ngroups, const 
         w.occ.ensure(1);
         return;
     }
-    check(hipMemsetAsync(w.occCount.p, 0, sizeof(int) * ncluster, s), "clear occurrences");
-    launchOccurrences(s, ngroups, groups, groupInfo, unionList, ncluster, w.occCount.p, nullptr, nullptr, false);
-    launchExclusiveScanWide(s, ncluster, w.occCount.p, w.occOff.p, w.occOff.p + ncluster);
-    int total = maxTotal;
-    if (total < 0)
+    if (!counted)
     {
-        int* const h = pinnedInts();
-        check(hipMemcpyAsync(h, w.occOff.p + ncluster, sizeof(int), hipMemcpyDeviceToHost, s), "read occurrences");
-        check(hipStreamSynchronize(s), "occurrence sync");
-        total = h[0];
+        check(hipMemsetAsync(w.occCount.p, 0, sizeof(int) * ncluster, s), "clear occurrences");
+        launchOccurrences(s, ngroups, groups, groupInfo, unionList, ncluster, w.occCount.p, nullptr, nullptr, false);
     }
-    w.occ.ensure(std::max(total, 1));
-    check(hipMemsetAsync(w.occCount.p, 0, sizeof(int) * ncluster, s), "clear occurrences");
+    launchExclusiveScanWide(s, ncluster, w.occCount.p, w.occOff.p, w.occOff.p + ncluster);
+    w.occ.ensure(std::max(maxTotal, 1));
     launchOccurrences(s, ngroups, groups, groupInfo, unionList, ncluster, w.occCount.p, w.occOff.p, w.occ.p, true);
     check(hipGetLastError(), "occurrence kernels");
 }
@@ -229,12 +224,9 @@ struct WorkLayout
     int            groupSize = 0, ngroups = 0, nchunk = 0, windowSlots = 0, nwork = 0;
     int            numBlocks = 0; // workgroups of kKernelWaves wavefronts (the schedule's wavefronts / 4)
     bool           spill     = false; // some union clusters lie beyond their window (global atomics)
-    DevBuf<int>    unionCount, chunkCount, workCount, overflow, unionOff, chunkOff, workOff, unionList;
+    DevBuf<int>    unionCount, spillCount, unionOff, spillOff, unionList;
     DevBuf<int4>   chunks, groups, groupInfo;
-    // the group pass's output at upper-bound bases, before compaction
-    DevBuf<int>    unionTmp;
-    DevBuf<int4>   chunksTmp;
-    DevBuf<uint2>  workTmp;
+    DevBuf<int>    unionTmp; // the unions at upper-bound bases
     DevBuf<float4> chunkShift;
     DevBuf<uint2>  work;
     DevBuf<int2>   waveStart; // static schedule: each wavefront's first chunk and its group
@@ -330,7 +322,8 @@ struct nbx_context
     int                 searchCapJ = 0;
     nbx::DevBuf<uint2>  searchJTmp;
     nbx::DevBuf<int4>   searchITmp;
-    nbx::DevBuf<int>    countJ, countI, offJ, offI, totals;
+    nbx::DevBuf<int>    countJ, countI, countW, offJ, offI, offW, totals;
+    int                 numWork = 0; // work entries: j-entries with every i-entry padded to whole tiles
     nbx::DevBuf<int4>   ientry;
     nbx::DevBuf<uint2>  jentry, jentryTmp;
     // the list as searched, kept by the first prune after a search (every

@@ -17,17 +17,18 @@
 //     the group's spare slot G + U, which the kernel never flushes, so the
 //     kernel reads whole tiles without bounds checks and no two lanes of a
 //     tile share a live slot,
-//   * work chunks: i-entries cut into pieces of at most kChunkEntries
-//     j-entries, {ci, shift | self << 8 | special << 9, work start, tiles};
-//     self marks the piece that carries the cluster's Ewald/RF self energy
-//     (first piece of the central entry, kernel_ref_outer.h:286-326),
-//     special counts its leading tiles that hold masked entries.
+//   * work chunks, one per i-entry: {ci, shift | self << 8 | special << 9,
+//     work start, tiles}; self marks the central entry, which carries the
+//     cluster's Ewald/RF self energy (kernel_ref_outer.h:286-326), special
+//     counts its leading tiles that hold masked entries.
 // The union comes from a bitmap over the range of the group's j-cluster
 // indices (one bit per cluster, set with LDS atomics; the per-word bit
 // counts scanned give each cluster's rank, so a j-entry's slot is one
 // popcount away), or from a bitonic sort of the keys when the range is wider
 // than the bitmap.
-// Like the search it runs as a count pass, a device scan, and a fill pass.
+// 288,000-atom water: the pass with its count, compaction, shift and cost
+// kernels and the search's compaction took 228 us (106 of them the pass), the
+// one pass and the union move take 136 us.
 #include <algorithm>
 #include <climits>
 
@@ -117,37 +118,119 @@ __device__ int blockExclusiveScan(int* v, int n, int* waveTot)
     return total;
 }
 
-template<bool kFill>
+// Measured cost of a chunk in the pair kernel, in 1/32 tile: 32 per tile,
+// plus 1.5 per tile for each i-atom whose type has LJ (the kernel skips the
+// LJ terms of the others), plus chunkCost per chunk (its set-up and i-force
+// reduction; kCostChunk of 19, 27 and 35: 163.6, 161.0 and 161.4 us for the
+// forces-only launch of the 288,000-atom water box).
+__device__ __forceinline__ int chunkCostOf(int tiles, int ci, const int* __restrict__ type,
+                                           const int* __restrict__ typeLJ, int chunkCost)
+{
+    int nlj = 0;
+#pragma unroll
+    for (int i = 0; i < kClusterSize; i++)
+    {
+        nlj += typeLJ[type[ci * kClusterSize + i]];
+    }
+    return tiles * (kCostTile + (3 * nlj) / 2) + chunkCost;
+}
+
+// One workgroup per group.  Everything but the union has its place from scans
+// over the clusters (i-entries, j-entries, padded work), so it is written once;
+// the unions, whose sizes are known only here, are moved together afterwards
+// (groupUnionsKernel).  Reads the list where the search left it.
 __global__ __launch_bounds__(kGroupThreads) void buildGroupsKernel(GroupArgs a)
 {
-    __shared__ int sKeys[kGroupMaxJ];
-    __shared__ int sFlag[kGroupMaxJ];
-    __shared__ int sUnion;
-    __shared__ int sChunks;
-    __shared__ int sWork;
-    __shared__ int sChunkBase[kGroupThreads];
-    __shared__ int sWorkBase[kGroupThreads];
-    __shared__ int sWaveTot[kGroupThreads / 64];
+    constexpr int kWaves = kGroupThreads / 64;
+    constexpr int kHeld  = 4; // j-entries per lane read together
+    static_assert(kGroupSizeMax * kMaxIEntriesPerCluster <= kGroupThreads, "a thread per i-entry of a group");
+    __shared__ int  sKeys[kGroupMaxJ];
+    __shared__ int  sFlag[kGroupMaxJ];
+    __shared__ int4 sEntry[kGroupThreads]; // i-entries {ci, shift, j start and end as read}
+    __shared__ int  sDst[kGroupThreads];   // their j start in the compact list
+    __shared__ int  sWorkBase[kGroupThreads];
+    __shared__ int  sWaveTot[kWaves];
+    __shared__ int  sMin[kWaves], sMax[kWaves];
+    __shared__ int  sOffI[kGroupSizeMax + 1], sOffJ[kGroupSizeMax + 1];
 
-    const int g  = blockIdx.x;
-    const int c0 = g * a.groupSize;
-    const int c1 = min(c0 + a.groupSize, a.ncluster);
-    const int jb = a.offJ[c0];
-    const int n  = a.offJ[c1] - jb;
-    const int ib = a.offI[c0];
-    const int ni = a.offI[c1] - ib;
-    // range of the group's other j-clusters: a bitmap over it (in sKeys)
+    const int g    = blockIdx.x;
+    const int c0   = g * a.groupSize;
+    const int c1   = min(c0 + a.groupSize, a.ncluster);
+    const int jb   = a.offJ[c0];
+    const int n    = a.offJ[c1] - jb;
+    const int ib   = a.offI[c0];
+    const int ni   = a.offI[c1] - ib;
+    const int woff = a.offW[c0];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+
+    if (static_cast<int>(threadIdx.x) <= c1 - c0)
+    {
+        sOffI[threadIdx.x] = a.offI[c0 + threadIdx.x];
+        sOffJ[threadIdx.x] = a.offJ[c0 + threadIdx.x];
+        if (static_cast<int>(threadIdx.x) < c1 - c0)
+        {
+            a.occCount[c0 + threadIdx.x] = 0;
+        }
+    }
+    __syncthreads();
+    // the group's i-entries, a thread each
+    {
+        const int e  = threadIdx.x;
+        int       nw = 0;
+        if (e < ni)
+        {
+            int k = 0; // its cluster in the group
+            while (c0 + k + 1 < c1 && sOffI[k + 1] - ib <= e)
+            {
+                k++;
+            }
+            const int  c  = c0 + k;
+            const int4 ie = a.ientryIn[a.capJ > 0 ? c * kMaxIEntriesPerCluster + (ib + e - sOffI[k]) : ib + e];
+            // j-entries move from the cluster's region to its scanned offset
+            const int dst        = a.capJ > 0 ? sOffJ[k] + (ie.z - c * a.capJ) : ie.z;
+            sEntry[e]            = ie;
+            sDst[e]              = dst;
+            nw                   = (ie.w - ie.z + kTileJ - 1) / kTileJ * kTileJ;
+            a.chunkShift[ib + e] = a.shiftVec[ie.y];
+            if (a.chunkCost)
+            {
+                a.chunkCost[ib + e] = chunkCostOf(nw / kTileJ, ie.x, a.type, a.typeLJ, kCostChunk);
+            }
+            if (a.capJ > 0)
+            {
+                a.ientryOut[ib + e] = make_int4(ie.x, ie.y, dst, dst + (ie.w - ie.z));
+            }
+        }
+        sWorkBase[e] = nw;
+    }
+    blockExclusiveScan(sWorkBase, kGroupThreads, sWaveTot); // (ends with a barrier)
+
+    // range of the group's j-clusters: a bitmap over it (in sKeys)
     // gives the sorted union and each cluster's rank directly; a range
     // wider than the bitmap takes a bitonic sort of the keys instead
-    __shared__ int sMin[kGroupThreads / 64], sMax[kGroupThreads / 64];
     int lo = INT_MAX, hi = -1;
-    for (int t = threadIdx.x; t < n; t += kGroupThreads)
+    if (a.capJ > 0)
     {
-        const int cj = static_cast<int>(a.jentryIn[jb + t].x);
-        if (cj < c0 || cj >= c1)
+        // as searched, an i-entry's j-clusters ascend
+        if (static_cast<int>(threadIdx.x) < ni)
         {
-            lo = min(lo, cj);
-            hi = max(hi, cj);
+            const int4 ie = sEntry[threadIdx.x];
+            lo            = static_cast<int>(a.jentryIn[ie.z].x);
+            hi            = static_cast<int>(a.jentryIn[ie.w - 1].x);
+        }
+    }
+    else
+    {
+        for (int e = wave; e < ni; e += kWaves)
+        {
+            const int4 ie = sEntry[e];
+            for (int t = ie.z + lane; t < ie.w; t += 64)
+            {
+                const int cj = static_cast<int>(a.jentryIn[t].x);
+                lo           = min(lo, cj);
+                hi           = max(hi, cj);
+            }
         }
     }
 #pragma unroll
@@ -156,14 +239,14 @@ __global__ __launch_bounds__(kGroupThreads) void buildGroupsKernel(GroupArgs a)
         lo = min(lo, __shfl_xor(lo, m, 64));
         hi = max(hi, __shfl_xor(hi, m, 64));
     }
-    if ((threadIdx.x & 63) == 0)
+    if (lane == 0)
     {
-        sMin[threadIdx.x >> 6] = lo;
-        sMax[threadIdx.x >> 6] = hi;
+        sMin[wave] = lo;
+        sMax[wave] = hi;
     }
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < kGroupThreads / 64; w++)
+    for (int w = 0; w < kWaves; w++)
     {
         lo = min(lo, sMin[w]);
         hi = max(hi, sMax[w]);
@@ -179,12 +262,26 @@ __global__ __launch_bounds__(kGroupThreads) void buildGroupsKernel(GroupArgs a)
             bm[w] = 0u;
         }
         __syncthreads();
-        for (int t = threadIdx.x; t < n; t += kGroupThreads)
+        for (int e = wave; e < ni; e += kWaves)
         {
-            const int cj = static_cast<int>(a.jentryIn[jb + t].x);
-            if (cj < c0 || cj >= c1)
+            const int4 ie = sEntry[e];
+            for (int t0 = ie.z; t0 < ie.w; t0 += 64 * kHeld)
             {
-                atomicOr(bm + ((cj - lo) >> 5), 1u << ((cj - lo) & 31));
+                int cj[kHeld];
+#pragma unroll
+                for (int u = 0; u < kHeld; u++)
+                {
+                    const int t = t0 + 64 * u + lane;
+                    cj[u]       = t < ie.w ? static_cast<int>(a.jentryIn[t].x) : c0;
+                }
+#pragma unroll
+                for (int u = 0; u < kHeld; u++)
+                {
+                    if (cj[u] < c0 || cj[u] >= c1)
+                    {
+                        atomicOr(bm + ((cj[u] - lo) >> 5), 1u << ((cj[u] - lo) & 31));
+                    }
+                }
             }
         }
         __syncthreads();
@@ -202,15 +299,18 @@ __global__ __launch_bounds__(kGroupThreads) void buildGroupsKernel(GroupArgs a)
         {
             p <<= 1;
         }
-        for (int t = threadIdx.x; t < p; t += kGroupThreads)
+        for (int t = n + threadIdx.x; t < p; t += kGroupThreads)
         {
-            int key = INT_MAX;
-            if (t < n)
+            sKeys[t] = INT_MAX;
+        }
+        for (int e = wave; e < ni; e += kWaves)
+        {
+            const int4 ie = sEntry[e];
+            for (int t = ie.z + lane; t < ie.w; t += 64)
             {
-                const int cj = static_cast<int>(a.jentryIn[jb + t].x);
-                key          = (cj >= c0 && cj < c1) ? INT_MAX : cj;
+                const int cj                   = static_cast<int>(a.jentryIn[t].x);
+                sKeys[sDst[e] - jb + t - ie.z] = (cj >= c0 && cj < c1) ? INT_MAX : cj;
             }
-            sKeys[t] = key;
         }
         __syncthreads();
         bitonicSort(sKeys, p);
@@ -222,56 +322,14 @@ __global__ __launch_bounds__(kGroupThreads) void buildGroupsKernel(GroupArgs a)
         }
         __syncthreads();
     }
-    // the group's i-entries (at most kGroupThreads; more is flagged as
-    // overflow below): their chunk counts and padded work lengths
-    {
-        const int e = threadIdx.x;
-        int       nc = 0, nw = 0;
-        if (e < ni)
-        {
-            const int4 ie = a.ientry[ib + e];
-            nc            = (ie.w - ie.z + a.chunkEntries - 1) / a.chunkEntries;
-            nw            = (ie.w - ie.z + kTileJ - 1) / kTileJ * kTileJ;
-        }
-        sChunkBase[e] = nc;
-        sWorkBase[e]  = nw;
-    }
-    // exclusive scans: ranks of the unique keys, and the chunk and padded
-    // work offsets of the i-entries
-    const int unionTotal = blockExclusiveScan(sFlag, bitmap ? nwords : p, sWaveTot);
-    const int chunkTotal = blockExclusiveScan(sChunkBase, kGroupThreads, sWaveTot);
-    const int workTotal  = blockExclusiveScan(sWorkBase, kGroupThreads, sWaveTot);
+    const int U = blockExclusiveScan(sFlag, bitmap ? nwords : p, sWaveTot);
+    // union clusters that get a window slot (the rest overflow)
+    const int Uw = min(U, a.windowCap - 1 - a.groupSize);
     if (threadIdx.x == 0)
     {
-        sUnion  = unionTotal;
-        sChunks = chunkTotal;
-        sWork   = workTotal;
+        a.unionCount[g] = U;
+        a.spillCount[g] = U - Uw;
     }
-    __syncthreads();
-    const int U      = sUnion;
-    // union clusters that get a window slot (the rest overflow)
-    const int Uw     = kFill ? min(U, a.windowCap - 1 - a.groupSize) : U;
-    const int nchunk = sChunks;
-    if (!kFill || a.upperBound)
-    {
-        if (threadIdx.x == 0)
-        {
-            a.unionCount[g] = U;
-            a.chunkCount[g] = nchunk;
-            a.workCount[g]  = sWork;
-            a.overflow[g]   = (ni > kGroupThreads) ? 1 : 0;
-        }
-        if (!kFill || ni > kGroupThreads)
-        {
-            return;
-        }
-    }
-    // where the group's union, chunks and work go: the scanned offsets, or
-    // (upperBound) bounds that need no scan of other groups: the union has
-    // at most n entries, the chunks (one per i-entry) at most ni, the padded
-    // work at most n + (kTileJ - 1) ni, so bases from the cluster offsets
-    // never overlap; groupCompactKernel moves them together afterwards
-    const int uoff = a.upperBound ? jb : a.unionOff[g];
     if (bitmap)
     {
         for (int w = threadIdx.x; w < nwords; w += kGroupThreads)
@@ -279,7 +337,7 @@ __global__ __launch_bounds__(kGroupThreads) void buildGroupsKernel(GroupArgs a)
             int r = sFlag[w];
             for (unsigned bits = bm[w]; bits; bits &= bits - 1u)
             {
-                a.unionList[uoff + r++] = lo + 32 * w + (__ffs(bits) - 1);
+                a.unionTmp[jb + r++] = lo + 32 * w + (__ffs(bits) - 1);
             }
         }
     }
@@ -290,169 +348,176 @@ __global__ __launch_bounds__(kGroupThreads) void buildGroupsKernel(GroupArgs a)
             const int k = sKeys[t];
             if (k != INT_MAX && (t == 0 || sKeys[t - 1] != k))
             {
-                a.unionList[uoff + sFlag[t]] = k;
+                a.unionTmp[jb + sFlag[t]] = k;
             }
         }
         __syncthreads();
         for (int t = threadIdx.x; t < U; t += kGroupThreads)
         {
-            sKeys[t] = a.unionList[uoff + t];
+            sKeys[t] = a.unionTmp[jb + t];
         }
     }
     __syncthreads();
-    const int coff = a.upperBound ? ib : a.chunkOff[g];
-    if (threadIdx.x == 0)
-    {
-        a.groups[g]    = make_int4(coff, coff + nchunk, uoff, Uw);
-        a.groupInfo[g] = make_int4(c0, (c1 - c0) | (a.groupSize << 16), 0, g);
-    }
-    // per i-entry: masked-first partition, slots, work list, chunks (one
+    // per i-entry: masked-first partition, slots, work list, chunk (one
     // wave per entry)
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int woff = a.upperBound ? jb + (kTileJ - 1) * ib : a.workOff[g];
-    for (int e = wave; e < ni; e += kGroupThreads / 64)
+    for (int e = wave; e < ni; e += kWaves)
     {
-        const int4 ie      = a.ientry[ib + e];
+        const int4 ie      = sEntry[e];
+        const int  dst     = sDst[e];
         const int  ci      = ie.x;
         const int  shift   = ie.y;
         const int  js      = ie.z;
         const int  je      = ie.w;
         const int  wb      = woff + sWorkBase[e];
-        int        written = 0;
-        int        nmasked = 0;
-        for (int pass = 0; pass < 2; pass++)
-        {
-            for (int t0 = js; t0 < je; t0 += 64)
+        // one entry to its place in the list and the work list
+        auto put = [&](const uint2 ent, int at) {
+            const int cj = static_cast<int>(ent.x);
+            int       slot;
+            if (cj >= c0 && cj < c1)
             {
-                const int  t    = t0 + lane;
-                uint2      ent  = make_uint2(0u, 0u);
-                bool       take = false;
-                if (t < je)
+                slot = cj - c0;
+            }
+            else
+            {
+                // the cluster's rank in the sorted union
+                int l;
+                if (bitmap)
                 {
-                    ent               = a.jentryIn[t];
-                    const bool masked = (ent.y & 0xffffu) != 0xffffu;
-                    take              = (pass == 0) ? masked : !masked;
+                    const int d = cj - lo;
+                    l           = sFlag[d >> 5] + __popc(bm[d >> 5] & ((1u << (d & 31)) - 1u));
                 }
-                const unsigned long long ballot = __ballot(take);
-                const int before = __popcll(ballot & ((1ull << lane) - 1ull));
-                if (take)
+                else
                 {
-                    const int cj = static_cast<int>(ent.x);
-                    int       slot;
-                    if (cj >= c0 && cj < c1)
+                    l     = 0;
+                    int r = U;
+                    while (l < r)
                     {
-                        slot = cj - c0;
-                    }
-                    else
-                    {
-                        // the cluster's rank in the sorted union
-                        int l;
-                        if (bitmap)
+                        const int m = (l + r) >> 1;
+                        if (sKeys[m] < cj)
                         {
-                            const int d = cj - lo;
-                            l           = sFlag[d >> 5] + __popc(bm[d >> 5] & ((1u << (d & 31)) - 1u));
+                            l = m + 1;
                         }
                         else
                         {
-                            l     = 0;
-                            int r = U;
-                            while (l < r)
-                            {
-                                const int m = (l + r) >> 1;
-                                if (sKeys[m] < cj)
-                                {
-                                    l = m + 1;
-                                }
-                                else
-                                {
-                                    r = m;
-                                }
-                            }
+                            r = m;
                         }
-                        slot = l < Uw ? a.groupSize + l : static_cast<int>(kSlotOverflow);
                     }
-                    a.jentryOut[js + written + before] = ent;
-                    a.work[wb + written + before] =
-                            make_uint2(ent.x, (static_cast<unsigned>(slot) << 16) | (ent.y & 0xffffu));
                 }
-                written += __popcll(ballot);
+                slot = l < Uw ? a.groupSize + l : static_cast<int>(kSlotOverflow);
             }
-            if (pass == 0)
+            a.jentryOut[dst + at] = ent;
+            a.work[wb + at]       = make_uint2(ent.x, (static_cast<unsigned>(slot) << 16) | (ent.y & 0xffffu));
+        };
+        const unsigned long long below   = (1ull << lane) - 1ull;
+        int                      nmasked = 0;
+        if (je - js <= 64 * kHeld)
+        {
+            // read once and held: the masked entries' places, then the others'
+            uint2              ent[kHeld];
+            unsigned long long masked[kHeld];
+#pragma unroll
+            for (int u = 0; u < kHeld; u++)
             {
-                nmasked = written;
+                const int t = js + 64 * u + lane;
+                ent[u]      = t < je ? a.jentryIn[t] : make_uint2(0u, 0xffffu);
+            }
+#pragma unroll
+            for (int u = 0; u < kHeld; u++)
+            {
+                masked[u] = __ballot((ent[u].y & 0xffffu) != 0xffffu);
+                nmasked += __popcll(masked[u]);
+            }
+            int atMasked = 0, atPlain = nmasked;
+#pragma unroll
+            for (int u = 0; u < kHeld; u++)
+            {
+                const int                here  = min(64, je - js - 64 * u); // entries of this part
+                const bool               mine  = lane < here;
+                const bool               isMsk = (masked[u] >> lane) & 1ull;
+                const unsigned long long plain = here >= 64 ? ~masked[u] : (here > 0 ? ~masked[u] & ((1ull << here) - 1ull) : 0ull);
+                if (mine)
+                {
+                    put(ent[u], isMsk ? atMasked + __popcll(masked[u] & below) : atPlain + __popcll(plain & below));
+                }
+                atMasked += __popcll(masked[u]);
+                atPlain += __popcll(plain);
+            }
+        }
+        else
+        {
+            int written = 0;
+            for (int pass = 0; pass < 2; pass++)
+            {
+                for (int t0 = js; t0 < je; t0 += 64)
+                {
+                    const int  t    = t0 + lane;
+                    uint2      ent  = make_uint2(0u, 0u);
+                    bool       take = false;
+                    if (t < je)
+                    {
+                        ent               = a.jentryIn[t];
+                        const bool masked = (ent.y & 0xffffu) != 0xffffu;
+                        take              = (pass == 0) ? masked : !masked;
+                    }
+                    const unsigned long long ballot = __ballot(take);
+                    if (take)
+                    {
+                        put(ent, written + __popcll(ballot & below));
+                    }
+                    written += __popcll(ballot);
+                }
+                if (pass == 0)
+                {
+                    nmasked = written;
+                }
             }
         }
         // pad to whole tiles with the dummy cluster, in the spare slot
-        const int n    = je - js;
-        const int npad = (n + kTileJ - 1) / kTileJ * kTileJ;
-        if (n + lane < npad)
+        const int len   = je - js;
+        const int tiles = (len + kTileJ - 1) / kTileJ;
+        if (len + lane < tiles * kTileJ)
         {
-            a.work[wb + n + lane] = make_uint2(static_cast<unsigned>(a.ncluster),
-                                               (static_cast<unsigned>(a.groupSize + Uw) << 16) | 0xffffu);
+            a.work[wb + len + lane] = make_uint2(static_cast<unsigned>(a.ncluster),
+                                                 (static_cast<unsigned>(a.groupSize + Uw) << 16) | 0xffffu);
         }
         if (lane == 0)
         {
-            const int base = coff + sChunkBase[e];
-            int       k    = 0;
-            for (int s = 0; s < n; s += a.chunkEntries, k++)
-            {
-                const int self  = (shift == kCentral && k == 0) ? 1 : 0;
-                const int tiles = (min(a.chunkEntries, n - s) + kTileJ - 1) / kTileJ;
-                // tiles of this chunk holding masked entries (they lead the list)
-                const int left    = max(0, nmasked - s);
-                const int special = min((left + kTileJ - 1) / kTileJ, tiles);
-                a.chunks[base + k] = make_int4(ci, shift | (self << 8) | (special << 9), wb + s, tiles);
-            }
+            const int self = shift == kCentral ? 1 : 0;
+            // tiles holding masked entries (they lead the list)
+            const int special = (nmasked + kTileJ - 1) / kTileJ;
+            a.chunks[ib + e]  = make_int4(ci, shift | (self << 8) | (special << 9), wb, tiles);
         }
     }
 }
 
-// The layout written at the upper-bound bases moved to its scanned
-// offsets (one workgroup per group): union, work entries and chunks, the
-// chunks' work starts and the group record rebased.  With a window of
-// a.windowCap slots, union clusters beyond it take kSlotOverflow and the
-// padding entries the spare slot after the last windowed one.
-__global__ __launch_bounds__(kGroupThreads) void groupCompactKernel(GroupArgs a, const int* __restrict__ unionTmp,
-                                                                    const uint2* __restrict__ workTmp,
-                                                                    const int4* __restrict__ chunksTmp)
+// The unions at their scanned offsets and the group records (one workgroup
+// per group), and the occurrences of every cluster in the groups' windows.
+__global__ __launch_bounds__(kGroupThreads) void groupUnionsKernel(GroupArgs a)
 {
     const int g  = blockIdx.x;
     const int c0 = g * a.groupSize;
+    const int c1 = min(c0 + a.groupSize, a.ncluster);
     const int jb = a.offJ[c0];
-    const int ib = a.offI[c0];
-    const int wb = jb + (kTileJ - 1) * ib;
-    const int U = a.unionCount[g], nch = a.chunkCount[g], nw = a.workCount[g];
-    const int uo = a.unionOff[g], co = a.chunkOff[g], wo = a.workOff[g];
+    const int U  = a.unionCount[g];
+    const int uo = a.unionOff[g];
     const int Uw = min(U, a.windowCap - 1 - a.groupSize);
-    const unsigned firstOver = static_cast<unsigned>(a.groupSize + Uw);
     for (int t = threadIdx.x; t < U; t += kGroupThreads)
     {
-        a.unionList[uo + t] = unionTmp[jb + t];
-    }
-    for (int t = threadIdx.x; t < nw; t += kGroupThreads)
-    {
-        uint2          e    = workTmp[wb + t];
-        const unsigned slot = e.y >> 16;
-        if (static_cast<int>(e.x) == a.ncluster)
+        const int cj        = a.unionTmp[jb + t];
+        a.unionList[uo + t] = cj;
+        if (t < Uw)
         {
-            e.y = (firstOver << 16) | (e.y & 0xffffu);
+            atomicAdd(a.occCount + cj, 1);
         }
-        else if (slot >= firstOver && slot != kSlotOverflow)
-        {
-            e.y = (kSlotOverflow << 16) | (e.y & 0xffffu);
-        }
-        a.work[wo + t] = e;
     }
-    for (int t = threadIdx.x; t < nch; t += kGroupThreads)
+    if (static_cast<int>(threadIdx.x) < c1 - c0)
     {
-        int4 c         = chunksTmp[ib + t];
-        c.z            = wo + (c.z - wb);
-        a.chunks[co + t] = c;
+        atomicAdd(a.occCount + c0 + threadIdx.x, 1);
     }
     if (threadIdx.x == 0)
     {
-        a.groups[g] = make_int4(co, co + nch, uo, Uw);
+        a.groups[g]    = make_int4(a.offI[c0], a.offI[c1], uo, Uw);
+        a.groupInfo[g] = make_int4(c0, (c1 - c0) | (a.groupSize << 16), 0, g);
     }
 }
 
@@ -538,7 +603,8 @@ __global__ void occurrenceKernel(int ngroups, const int4* __restrict__ groups, c
     for (int t = threadIdx.x; t < nOwn + grp.w; t += blockDim.x)
     {
         const int c = t < nOwn ? gi.x + t : unionList[grp.z + t - nOwn];
-        const int k = atomicAdd(&count[c], 1);
+        // the fill takes its places from the counts, downwards
+        const int k = kFill ? atomicSub(&count[c], 1) - 1 : atomicAdd(&count[c], 1);
         if (kFill)
         {
             occ[occOff[c] + k] = make_int2(g, t < nOwn ? t : G + (t - nOwn));
@@ -866,35 +932,13 @@ __global__ void segmentBaseKernel(int ngroups, const int* __restrict__ base, int
     }
 }
 
-__global__ void chunkShiftKernel(int nchunk, const int4* __restrict__ chunks, const float4* __restrict__ shiftVec,
-                                 float4* __restrict__ out)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nchunk)
-    {
-        out[k] = shiftVec[chunks[k].y & 0xff];
-    }
-}
-
-// Measured cost of a chunk in the pair kernel, in 1/32 tile: 32 per tile,
-// plus 1.5 per tile for each i-atom whose type has LJ (the kernel skips the
-// LJ terms of the others), plus 27 per chunk (its set-up and i-force
-// reduction).  Fitted to the run times of individual wavefronts on the
-// 288,000-atom water box, where it leaves 2.3 us of 205 us unexplained.
 __global__ void chunkCostKernel(int nchunk, const int4* __restrict__ chunks, const int* __restrict__ type,
                                 const int* __restrict__ typeLJ, int chunkCost, int* __restrict__ cost)
 {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m < nchunk)
     {
-        const int4 cd  = chunks[m];
-        int        nlj = 0;
-#pragma unroll
-        for (int i = 0; i < kClusterSize; i++)
-        {
-            nlj += typeLJ[type[cd.x * kClusterSize + i]];
-        }
-        cost[m] = cd.w * (kCostTile + (3 * nlj) / 2) + chunkCost;
+        cost[m] = chunkCostOf(chunks[m].w, chunks[m].x, type, typeLJ, chunkCost);
     }
 }
 
@@ -1142,14 +1186,6 @@ void launchGatherList(hipStream_t s, int ncluster, const int* occOff, const int2
     }
 }
 
-void launchChunkShifts(hipStream_t s, int nchunk, const int4* chunks, const float4* shiftVec, float4* out)
-{
-    if (nchunk > 0)
-    {
-        chunkShiftKernel<<<(nchunk + 255) / 256, 256, 0, s>>>(nchunk, chunks, shiftVec, out);
-    }
-}
-
 void launchWaveSchedule(hipStream_t s, int numWaves, int nchunk, const int4* chunks, int nwork, int chunkWeight,
                         int ngroups, const int4* groups, int2* out, const int* costOff, const int* costTotal,
                         int genWaves)
@@ -1174,28 +1210,19 @@ void launchSystemSlots(hipStream_t s, int numSystems, const int* groupOff, int n
                                                              waveStart, slotOff);
 }
 
-void launchGroupCompact(hipStream_t s, const GroupArgs& a, const int* unionTmp, const uint2* workTmp,
-                        const int4* chunksTmp)
+void launchBuildGroups(hipStream_t s, const GroupArgs& a)
 {
     if (a.ngroups > 0)
     {
-        groupCompactKernel<<<a.ngroups, kGroupThreads, 0, s>>>(a, unionTmp, workTmp, chunksTmp);
+        buildGroupsKernel<<<a.ngroups, kGroupThreads, 0, s>>>(a);
     }
 }
 
-void launchBuildGroups(hipStream_t s, const GroupArgs& a, bool fill)
+void launchGroupUnions(hipStream_t s, const GroupArgs& a)
 {
-    if (a.ngroups == 0)
+    if (a.ngroups > 0)
     {
-        return;
-    }
-    if (fill)
-    {
-        buildGroupsKernel<true><<<a.ngroups, kGroupThreads, 0, s>>>(a);
-    }
-    else
-    {
-        buildGroupsKernel<false><<<a.ngroups, kGroupThreads, 0, s>>>(a);
+        groupUnionsKernel<<<a.ngroups, kGroupThreads, 0, s>>>(a);
     }
 }
 

@@ -56,10 +56,8 @@ __device__ __forceinline__ float canonicalD2(float dx, float dy, float dz)
 // candidate group sizes: kGroupSizeMax, kGroupSizeMax / 2, ..., 1
 constexpr int kGroupSizeCount = 5;
 constexpr int kGroupMaxJ    = 4096;
-// j-clusters per kernel tile, j-entries per work chunk (a multiple of it;
-// large enough that a chunk is a whole i-entry)
-constexpr int kTileJ        = 16;
-constexpr int kChunkEntries = 1 << 20;
+// j-clusters per kernel tile (a work chunk is a whole i-entry)
+constexpr int kTileJ = 16;
 // cost of one chunk (i-entry) in work entries for the static schedule: its
 // i-data set-up and i-force reduction (64 replicas of 3,000 to 48,000 atoms:
 // 1016, 939 and 980 us per step with 8, 14 and 32)
@@ -241,6 +239,7 @@ struct SearchArgs
     // outputs (count pass writes counts; fill pass writes the lists)
     int*   countJ;   // per ci: number of j entries
     int*   countI;   // per ci: number of i entries
+    int*   countW;   // per ci: work entries (every i-entry padded to whole tiles)
     const int* offJ; // per ci: first j entry (exclusive scan of countJ)
     const int* offI; // per ci: first i entry
     int4*  ientry;
@@ -253,9 +252,8 @@ struct SearchArgs
 // shift indices at or below the central one: at most 14 i-entries per cluster
 constexpr int kMaxIEntriesPerCluster = 14;
 void launchSearch(hipStream_t s, const SearchArgs& a, bool fill);
-void launchSearchCompact(hipStream_t s, int ncluster, int capJ, const int* countJ, const int* countI,
-                         const int* offJ, const int* offI, const uint2* jentryTmp, const int4* ientryTmp,
-                         uint2* jentry, int4* ientry);
+// countW of a list's clusters from its i-entries (offI: ncluster + 1)
+void launchClusterWork(hipStream_t s, int ncluster, const int* offI, const int4* ientry, int* countW);
 void launchExclusiveScan(hipStream_t s, int n, const int* in, int* out, int* total);
 // count (at most 3) independent scans of n elements each in one launch, one
 // workgroup each
@@ -283,32 +281,39 @@ struct GroupArgs
     int          ncluster;
     int          groupSize;
     int          ngroups;
-    int          chunkEntries;
-    const int*   offI;      // per cluster: first i-entry (ncluster + 1)
-    const int*   offJ;      // per cluster: first j-entry (ncluster + 1)
-    const int4*  ientry;    // search output {ci, shift, cj_start, cj_end}
-    const uint2* jentryIn;  // search output {cj, mask}
-    uint2*       jentryOut; // the same entries, masked entries first
-    int*         unionCount; // count pass, per group
-    int*         chunkCount; // count pass, per group
-    int*         workCount;  // count pass, per group: padded work entries
-    int*         overflow;   // count pass, per group
-    const int*   unionOff;   // fill pass: exclusive scan of unionCount
-    const int*   chunkOff;   // fill pass: exclusive scan of chunkCount
-    const int*   workOff;    // fill pass: exclusive scan of workCount
-    int*         unionList;
+    // per cluster, exclusive scans (ncluster + 1): i-entries, j-entries and
+    // padded work entries
+    const int*   offI;
+    const int*   offJ;
+    const int*   offW;
+    // the list: i-entries {ci, shift, cj_start, cj_end} and j-entries {cj,
+    // mask}, compact (capJ = 0) or as the search left them, cluster c's at
+    // ientryIn[c * kMaxIEntriesPerCluster] and jentryIn[c * capJ]
+    const int4*  ientryIn;
+    const uint2* jentryIn;
+    int          capJ;
+    int4*        ientryOut;  // capJ > 0: the compact i-entries
+    uint2*       jentryOut;  // the compact j-entries, masked entries first
+    int*         unionCount; // per group
+    int*         spillCount; // per group: union clusters beyond the window
+    int*         unionTmp;   // unions at offJ[first cluster], for launchGroupUnions
     uint2*       work;       // {cj, slot << 16 | mask}, each chunk padded to whole tiles
-    int4*        chunks;     // {ci, shift | self << 8 | special << 9, work_start, tiles}
-    int4*        groups;     // {chunk_start, chunk_end, union_offset, union_size}
-    int4*        groupInfo;  // {first own cluster, own count | G << 16, shift-table offset, group index}
-    int          windowCap;  // fill pass: window slots (own, union, spare); union beyond -> kSlotOverflow
-    // fill pass without a count pass: writes the per-group counts and the
-    // layout at upper-bound bases (union at offJ[c0], chunks at offI[c0],
-    // work at offJ[c0] + (kTileJ - 1) offI[c0]) for launchGroupCompact
-    int          upperBound;
+    int4*        chunks;     // per i-entry: {ci, shift | self << 8 | special << 9, work start, tiles}
+    float4*      chunkShift; // per chunk: its shift vector
+    const float4* shiftVec;
+    int*         chunkCost;  // per chunk, when given: launchChunkCosts' cost from type, typeLJ
+    const int*   type;
+    const int*   typeLJ;
+    int          windowCap;  // window slots (own, union, spare); union beyond -> kSlotOverflow
     // 1: every group's union by a bitonic sort of its keys (the path taken
     // by groups whose j-clusters span more than the bitmap covers), for tests
     int          unionBySort;
+    // launchGroupUnions
+    const int*   unionOff;   // exclusive scan of unionCount
+    int*         unionList;
+    int4*        groups;     // {chunk_start, chunk_end, union_offset, union_size}
+    int4*        groupInfo;  // {first own cluster, own count | G << 16, shift-table offset, group index}
+    int*         occCount;   // per cluster: occurrences in the groups' windows (zeroed by launchBuildGroups)
 };
 // window slot of a j-entry whose cluster did not fit the group's window:
 // the kernel adds its forces with global atomics
@@ -318,11 +323,10 @@ constexpr unsigned kSlotOverflow = 0xffffu;
 // on the order of the atomics, so the sums are reproducible.  Resolution
 // 2^-20 (about 1e-6 kJ mol^-1 nm^-1), range +-2^43 (about 8.8e12).
 constexpr int kFixBits = 20;
-void launchBuildGroups(hipStream_t s, const GroupArgs& a, bool fill);
-// moves an upper-bound layout (unionTmp, workTmp, chunksTmp) to a.unionOff,
-// a.workOff, a.chunkOff in a.unionList, a.work, a.chunks; rebases a.groups
-void launchGroupCompact(hipStream_t s, const GroupArgs& a, const int* unionTmp, const uint2* workTmp,
-                        const int4* chunksTmp);
+void launchBuildGroups(hipStream_t s, const GroupArgs& a);
+// after the scan of unionCount: the unions at their offsets, the group
+// records, and every cluster's occurrence count
+void launchGroupUnions(hipStream_t s, const GroupArgs& a);
 // Maxima for buffer sizing, as per-workgroup partials that the host reads
 // and reduces (reducePartialMax): of nv (at most 2) arrays of n non-negative
 // ints, and with offJ (the scanned j-entry counts of n clusters) of the
@@ -347,9 +351,9 @@ int  launchPartialMax(hipStream_t s, const PartialMaxArgs& a);
 void reducePartialMax(const int* partial, int blocks, int stride, int* out);
 // Occurrences of every cluster in the groups' j-force windows (own slot and
 // windowed-union slots) as a CSR list of {group, slot}, sorted per cluster.
-// Call once with fill = false (count must be zeroed; it returns the counts),
-// scan the counts into occOff[ncluster + 1], zero count, call with fill = true
-// (count holds ncluster + 1 ints; the fill's sort overwrites it).
+// Call once with fill = false (count must be zeroed; it returns the counts;
+// launchGroupUnions counts too), scan the counts into occOff[ncluster + 1],
+// call with fill = true (count, ncluster + 1 ints, is used up).
 void launchOccurrences(hipStream_t s, int ngroups, const int4* groups, const int4* groupInfo, const int* unionList,
                        int ncluster, int* count, int* occOff, int2* occ, bool fill);
 // The pair kernel's window staging layout for a schedule: per group
@@ -364,9 +368,6 @@ void launchSegments(hipStream_t s, int ngroups, const int4* groups, const int4* 
 // then fill.
 void launchGatherList(hipStream_t s, int ncluster, const int* occOff, const int2* occ, const int4* segInfo,
                       int slotF4, int* count, const int* gposOff, int* gpos, bool fill);
-// Per chunk, the shift vector of its i-entry (shiftVec[chunk shift index]),
-// so that the pair kernel loads it together with the chunk descriptor.
-void launchChunkShifts(hipStream_t s, int nchunk, const int4* chunks, const float4* shiftVec, float4* out);
 // Static schedule of the pair kernel: the chunk list (in group order) cut into
 // numWaves contiguous runs of about equal cost (the exclusive scan costOff of
 // launchChunkCosts' per-chunk costs, total *costTotal, when costOff is given;

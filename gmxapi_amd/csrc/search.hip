@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kWave* kSearchWaves) __attribute__((amdgpu_waves_pe
     {
         // capJ > 0: a fill without a count pass, into this cluster's own
         // region of capJ j-entries and kMaxIEntriesPerCluster i-entries
-        // (searchCompactKernel moves them together after the scans)
+        // (the group pass moves them together after the scans)
         jpos = a.capJ > 0 ? ci * a.capJ : a.offJ[ci];
         ipos = a.capJ > 0 ? ci * kMaxIEntriesPerCluster : a.offI[ci];
         int cnt[kClusterSize], beg[kClusterSize];
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(kWave* kSearchWaves) __attribute__((amdgpu_waves_pe
             }
         }
     }
-    int countJ = 0, countI = 0;
+    int countJ = 0, countI = 0, countW = 0;
     const float4 bbLo = make_float4(uniformF(lo.x), uniformF(lo.y), uniformF(lo.z), 0.0f);
     const float4 bbHi = make_float4(uniformF(hi.x), uniformF(hi.y), uniformF(hi.z), 0.0f);
     // the shifts that leave the box within rlist of the cell, per direction
@@ -480,6 +480,7 @@ __global__ __launch_bounds__(kWave* kSearchWaves) __attribute__((amdgpu_waves_pe
                     }
                     countJ += entryJ;
                     countI += 1;
+                    countW += (entryJ + kTileJ - 1) / kTileJ * kTileJ;
                 }
             }
         }
@@ -488,36 +489,22 @@ __global__ __launch_bounds__(kWave* kSearchWaves) __attribute__((amdgpu_waves_pe
     {
         a.countJ[ci] = countJ;
         a.countI[ci] = countI;
+        a.countW[ci] = countW;
     }
 }
 
-// A capped fill's lists moved to the scanned offsets (one wavefront per
-// cluster), the i-entries' j ranges rebased.
-__global__ __launch_bounds__(256) void searchCompactKernel(int ncluster, int capJ, const int* __restrict__ countJ,
-                                                           const int* __restrict__ countI,
-                                                           const int* __restrict__ offJ, const int* __restrict__ offI,
-                                                           const uint2* __restrict__ jentryTmp,
-                                                           const int4* __restrict__ ientryTmp,
-                                                           uint2* __restrict__ jentry, int4* __restrict__ ientry)
+__global__ void clusterWorkKernel(int ncluster, const int* __restrict__ offI, const int4* __restrict__ ientry,
+                                  int* __restrict__ countW)
 {
-    const int lane = threadIdx.x & 63;
-    const int ci   = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (ci >= ncluster)
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < ncluster)
     {
-        return;
-    }
-    const int nJ = countJ[ci], nI = countI[ci];
-    const int src = ci * capJ, dst = offJ[ci];
-    for (int t = lane; t < nJ; t += 64)
-    {
-        jentry[dst + t] = jentryTmp[src + t];
-    }
-    if (lane < nI)
-    {
-        int4 ie = ientryTmp[ci * kMaxIEntriesPerCluster + lane];
-        ie.z    = dst + (ie.z - src);
-        ie.w    = dst + (ie.w - src);
-        ientry[offI[ci] + lane] = ie;
+        int work = 0;
+        for (int e = offI[c]; e < offI[c + 1]; e++)
+        {
+            work += (ientry[e].w - ientry[e].z + kTileJ - 1) / kTileJ * kTileJ;
+        }
+        countW[c] = work;
     }
 }
 
@@ -872,14 +859,11 @@ void launchSearch(hipStream_t s, const SearchArgs& a, bool fill)
     }
 }
 
-void launchSearchCompact(hipStream_t s, int ncluster, int capJ, const int* countJ, const int* countI,
-                         const int* offJ, const int* offI, const uint2* jentryTmp, const int4* ientryTmp,
-                         uint2* jentry, int4* ientry)
+void launchClusterWork(hipStream_t s, int ncluster, const int* offI, const int4* ientry, int* countW)
 {
     if (ncluster > 0)
     {
-        searchCompactKernel<<<(ncluster + 3) / 4, 256, 0, s>>>(ncluster, capJ, countJ, countI, offJ, offI, jentryTmp,
-                                                              ientryTmp, jentry, ientry);
+        clusterWorkKernel<<<(ncluster + 255) / 256, 256, 0, s>>>(ncluster, offI, ientry, countW);
     }
 }
 
