@@ -303,13 +303,10 @@ const float* deviceCoordinates(nbx_context* c, const float* x, int onDevice)
 }
 
 // The list build's sizing reads: kStatsHead ints of scan totals, then the
-// per-workgroup maxima of launchPartialMax, read back in one copy.
+// per-workgroup maxima of launchPartialMax, which the kernels write straight
+// to the calling thread's pinned buffer: one stream wait, no copies.
 constexpr int kStatsHead = 4;
 static_assert(kStatsHead + kPartialMaxBlocks * partialMaxStride(2, true) <= kPinnedInts, "stats fit the pinned buffer");
-static void ensureStats(nbx_context* c)
-{
-    c->statsPartial.ensure(kStatsHead + kPartialMaxBlocks * partialMaxStride(2, true));
-}
 
 // the forward kernel's schedule by the measured cost model (unless the cost
 // total could overflow an int)
@@ -369,13 +366,9 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
     }
     else
     {
-        ensureStats(c);
-        const PartialMaxArgs pm{ { nullptr, nullptr }, 0, c->offJ.p, nc, c->statsPartial.p + kStatsHead };
-        const int            nb = launchPartialMax(c->stream, pm);
         int* const           hp = pinnedInts();
-        check(hipMemcpyAsync(hp, c->statsPartial.p + kStatsHead, sizeof(int) * nb * kGroupSizeCount,
-                             hipMemcpyDeviceToHost, c->stream),
-              "read spans");
+        const PartialMaxArgs pm{ { nullptr, nullptr }, 0, c->offJ.p, nc, hp };
+        const int            nb = launchPartialMax(c->stream, pm);
         check(hipStreamSynchronize(c->stream), "group sync");
         reducePartialMax(hp, nb, kGroupSizeCount, spans);
     }
@@ -490,20 +483,16 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
         ga.occCount    = L.gather.occCount.p;
         launchBuildGroups(c->stream, ga);
         // the largest union, as per-workgroup maxima after the totals of the
-        // unions and of what lies beyond the windows (one read)
-        ensureStats(c);
-        const PartialMaxArgs pm{ { L.unionCount.p, nullptr }, 1, nullptr, ng, c->statsPartial.p + kStatsHead };
+        // unions and of what lies beyond the windows (one wait)
+        int* const           hp = pinnedInts();
+        const PartialMaxArgs pm{ { L.unionCount.p, nullptr }, 1, nullptr, ng, hp + kStatsHead };
         const int            statBlocks = launchPartialMax(c->stream, pm);
         {
             const int* in[2]  = { L.unionCount.p, L.spillCount.p };
             int*       out[2] = { L.unionOff.p, L.spillOff.p };
-            int*       tot[2] = { c->statsPartial.p, c->statsPartial.p + 1 };
+            int*       tot[2] = { hp, hp + 1 };
             launchExclusiveScansWide(c->stream, ng, 2, in, out, tot);
         }
-        int* const hp = pinnedInts();
-        check(hipMemcpyAsync(hp, c->statsPartial.p, sizeof(int) * (kStatsHead + statBlocks), hipMemcpyDeviceToHost,
-                             c->stream),
-              "read stats");
         check(hipStreamSynchronize(c->stream), "group sync");
         int maxUnion = 0;
         reducePartialMax(hp + kStatsHead, statBlocks, 1, &maxUnion);
@@ -1150,20 +1139,27 @@ int nbx_put_on_grid(nbx_context* c, const float* box, const float* x, int xOnDev
         const size_t maxCluster = static_cast<size_t>(n) / kClusterSize + g.ncol + 1;
         const size_t maxSlot    = maxCluster * kClusterSize;
 
-        // shift vectors (calc_shifts, pbc.cpp:1187-1202)
-        std::vector<float4> sv(kNumShifts);
-        for (int n_ = 0, m = -1; m <= 1; m++)
+        // shift vectors (calc_shifts, pbc.cpp:1187-1202), for a new box
+        if (!std::equal(box, box + 3, c->shiftBox))
         {
-            for (int l = -1; l <= 1; l++)
+            std::vector<float4> sv(kNumShifts);
+            for (int n_ = 0, m = -1; m <= 1; m++)
             {
-                for (int k = -2; k <= 2; k++, n_++)
+                for (int l = -1; l <= 1; l++)
                 {
-                    sv[n_] = make_float4(k * box[0], l * box[1], m * box[2], 0.0f);
+                    for (int k = -2; k <= 2; k++, n_++)
+                    {
+                        sv[n_] = make_float4(k * box[0], l * box[1], m * box[2], 0.0f);
+                    }
                 }
             }
+            c->shiftBox[0] = 0.0f; // none until the copy is done
+            check(hipMemcpyAsync(c->shiftVec.p, sv.data(), sizeof(float4) * kNumShifts, hipMemcpyHostToDevice,
+                                 c->stream),
+                  "upload shifts");
+            check(hipStreamSynchronize(c->stream), "sync");
+            std::copy(box, box + 3, c->shiftBox);
         }
-        check(hipMemcpyAsync(c->shiftVec.p, sv.data(), sizeof(float4) * kNumShifts, hipMemcpyHostToDevice, c->stream),
-              "upload shifts");
 
         const float* xd = deviceCoordinates(c, x, xOnDevice);
         if (xd != c->x.p)
@@ -1178,14 +1174,10 @@ int nbx_put_on_grid(nbx_context* c, const float* box, const float* x, int xOnDev
         c->cells.ensure(n);
         c->bucket.ensure(maxSlot);
         c->atomIndices.ensure(maxSlot);
-        c->counter.ensure(4);
         check(hipMemsetAsync(c->cxy_na.p, 0, sizeof(int) * (g.ncol + 1), c->stream), "clear counts");
         launchGridColumns(c->stream, g, c->x.p, c->atomCol.p, c->atomRank.p, c->cxy_na.p);
-        launchGridScan(c->stream, g.ncol, c->cxy_na.p, c->cxy_ind.p, c->counter.p);
         int* const hp = pinnedInts();
-        check(hipMemcpyAsync(hp, c->counter.p, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream), "read count");
-        check(hipMemcpyAsync(hp + 2, c->cxy_na.p + g.ncol, sizeof(int), hipMemcpyDeviceToHost, c->stream),
-              "read flag");
+        launchGridScan(c->stream, g.ncol, c->cxy_na.p, c->cxy_ind.p, hp);
         check(hipStreamSynchronize(c->stream), "grid sync");
         const int hostCounts[3] = { hp[0], hp[1], hp[2] };
         if (hostCounts[2] != 0)
@@ -1254,7 +1246,7 @@ int nbx_construct_pairlist(nbx_context* c)
         c->offI.ensure(scanOutSize(nc));
         c->offW.ensure(scanOutSize(nc));
         c->totals.ensure(3);
-        ensureStats(c);
+        int* const hp = pinnedInts();
         SearchArgs a{};
         a.g           = c->g;
         a.rlist       = c->rlist;
@@ -1276,7 +1268,7 @@ int nbx_construct_pairlist(nbx_context* c)
         auto scanCounts = [&] {
             const int* in[3]  = { c->countJ.p, c->countI.p, c->countW.p };
             int*       out[3] = { c->offJ.p, c->offI.p, c->offW.p };
-            int*       tot[3] = { c->statsPartial.p, c->statsPartial.p + 1, c->statsPartial.p + 2 };
+            int*       tot[3] = { hp, hp + 1, hp + 2 };
             launchExclusiveScansWide(c->stream, nc, 3, in, out, tot);
         };
         // the list's totals, its largest j-entry count and the group pass's
@@ -1285,18 +1277,13 @@ int nbx_construct_pairlist(nbx_context* c)
         int  spans[kGroupSizeCount] = {};
         int  statBlocks             = 0;
         auto readStats              = [&] {
-            constexpr int kStride = partialMaxStride(1, true);
-            const PartialMaxArgs pm{ { c->countJ.p, nullptr }, 1, c->offJ.p, nc, c->statsPartial.p + kStatsHead };
+            const PartialMaxArgs pm{ { c->countJ.p, nullptr }, 1, c->offJ.p, nc, hp + kStatsHead };
             statBlocks = launchPartialMax(c->stream, pm);
-            check(hipMemcpyAsync(pinnedInts(), c->statsPartial.p, sizeof(int) * (kStatsHead + statBlocks * kStride),
-                                 hipMemcpyDeviceToHost, c->stream),
-                  "read stats");
         };
         // after the wait: j- and i-entry totals and the largest j-entry count
         // in tot, the spans in spans
         auto takeReads = [&](int* tot) {
-            const int* hp = pinnedInts();
-            int        st[partialMaxStride(1, true)];
+            int st[partialMaxStride(1, true)];
             reducePartialMax(hp + kStatsHead, statBlocks, partialMaxStride(1, true), st);
             tot[0]     = hp[0];
             tot[1]     = hp[1];

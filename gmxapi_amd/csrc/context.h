@@ -42,10 +42,9 @@ inline void check(hipError_t e, const char* what)
 }
 
 // The calling thread's pinned host buffer (kPinnedInts ints, allocated on
-// first use and kept for the thread's life) for the list build's small
-// device-to-host reads: a copy into pageable memory waits for its own staging
-// copy, one into pinned memory is queued, so several reads share one
-// stream synchronisation.  Callers use disjoint ranges within one wait.
+// first use and kept for the thread's life) that the list build's kernels
+// write their totals to: read after one stream wait, no copies.  Callers
+// use disjoint ranges within one wait.
 constexpr int kPinnedInts = 1024;
 inline int* pinnedInts()
 {
@@ -186,10 +185,9 @@ inline void buildSegments(hipStream_t s, WindowGather& w, int ngroups, const int
     int total = 0;
     if (ngroups > 0)
     {
-        launchSegments(s, ngroups, groups, groupInfo, numWaves, waveStart, slotF4, w.segSize.p, w.segBase.p,
-                       w.segBase.p + ngroups, w.segInfo.p);
         int* const h = pinnedInts();
-        check(hipMemcpyAsync(h, w.segBase.p + ngroups, sizeof(int), hipMemcpyDeviceToHost, s), "read segments");
+        launchSegments(s, ngroups, groups, groupInfo, numWaves, waveStart, slotF4, w.segSize.p, w.segBase.p, h,
+                       w.segInfo.p);
         check(hipStreamSynchronize(s), "segment sync");
         total = h[0];
     }
@@ -294,6 +292,7 @@ struct nbx_context
     nbx::DevBuf<float4> tabFDV0;
     nbx::DevBuf<double> tabFDV0d;
     nbx::DevBuf<float4> shiftVec;
+    float               shiftBox[3] = { 0.0f, 0.0f, 0.0f }; // the box shiftVec is for (edges are positive)
 
     // topology
     int         natoms = -1;
@@ -310,7 +309,7 @@ struct nbx_context
     bool        gridValid = false;
     int         ncluster  = 0;
     nbx::DevBuf<float> x;          // device copy of coordinates in atom order
-    nbx::DevBuf<int>   cxy_na, cxy_ind, atomCol, atomRank, bucket, atomIndices, cells, nbtype, counter;
+    nbx::DevBuf<int>   cxy_na, cxy_ind, atomCol, atomRank, bucket, atomIndices, cells, nbtype;
     nbx::DevBuf<float4> xq, bb, fnb;
     nbx::DevBuf<unsigned long long> fixF; // window-overflow forces in fixed point, 3 per atom slot
 
@@ -336,7 +335,6 @@ struct nbx_context
     // kernel work layouts: the pair kernel's, and the adjoint's (its own
     // group size, sized for its larger window per cluster slot; built on
     // the first adjoint call after a search)
-    nbx::DevBuf<int>    statsPartial; // per-workgroup maxima (launchPartialMax)
     nbx::DevBuf<int>    typeLJ; // per type (padding type included): 1 if it has LJ with any type
     unsigned long long  ljMask = 0; // typeLJ as bits (at most kMaxTypes + 1 types)
     bool                anyTypeWithoutLJ = false; // among the user's types
