@@ -1561,7 +1561,6 @@ static void enqueueStep(nbx_context* c, unsigned flags, const float* xd, float* 
     if (energy)
     {
         ExclusionArgs& e = a.excl;
-        e.natoms         = c->natoms;
         e.nslot          = c->ncluster * kClusterSize;
         e.npairs         = c->numExclPairs;
         e.pairSlots      = c->exclPairSlots.p;

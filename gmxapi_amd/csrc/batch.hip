@@ -42,14 +42,19 @@ struct nbx_batch
 
     DevBuf<float4> xq, fnb, shiftVec, chunkShift;
     DevBuf<unsigned long long> fixF; // window-overflow forces in fixed point, 3 per atom slot
-    DevBuf<int>    nbtype, atomIndices, cells, exclOff, exclIdx, unionList, atomSystem, groupOff, atomOff, slotOff;
+    DevBuf<int>    nbtype, atomIndices, unionList, groupOff, exclBlockOff, exclBlockSystem, slotOff;
     DevBuf<int2>   waveStart;
     DevBuf<int>    chunkCost, costOff; // the schedule's per-chunk costs (and their total) and their scan
     DevBuf<float>  boxes;
     WindowGather   gather;
     DevBuf<uint2>  work;
     DevBuf<int4>   chunks, groups, groupInfo;
-    DevBuf<double> energyPartial, atomEnergy;
+    // the exclusion pass: excluded pairs as cluster slots, and its workgroups'
+    // {first slot, end, first pair, end}
+    DevBuf<int2>   exclPairSlots;
+    DevBuf<int4>   exclBlocks;
+    int            numExclBlocks = 0;
+    DevBuf<double> energyPartial, exclPartial;
     PinnedBuf<double> energy; // per system {LJ, Coulomb}, written by the step's final sums
     bool           haveEnergy = false;
 
@@ -180,9 +185,10 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
     check(hipSetDevice(b->device), "hipSetDevice");
 
     std::vector<float4> hXq;
-    std::vector<int>    hType, hAi, hCells, hExOff{ 0 }, hExIdx, hUnion, hAtomSys, hGroupOff{ 0 }, hAtomOff{ 0 };
+    std::vector<int>    hType, hAi, hUnion, hGroupOff{ 0 }, hExclOff{ 0 }, hExclSystem;
+    std::vector<int2>   hExclPairs;
     std::vector<uint2>  hWork;
-    std::vector<int4>   hChunks, hGroups, hInfo;
+    std::vector<int4>   hChunks, hGroups, hInfo, hExclBlocks;
     std::vector<float4> hShift, hChunkShift;
     int                 clusterOff = 0, atomOffset = 0, maxSlots = 0;
     bool                anySpill = false;
@@ -205,7 +211,6 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
         std::vector<float4> xq = download(c->xq.p, 4 * static_cast<size_t>(nc) + 4);
         std::vector<int>    ty = download(c->nbtype.p, 4 * static_cast<size_t>(nc) + 4);
         std::vector<int>    ai = download(c->atomIndices.p, 4 * static_cast<size_t>(nc));
-        std::vector<int>    ce = download(c->cells.p, na);
         std::vector<uint2>  wk = download(c->lay.work.p, c->lay.nwork);
         std::vector<int4>   ch = download(c->lay.chunks.p, c->lay.nchunk);
         std::vector<float4> cs = download(c->lay.chunkShift.p, c->lay.nchunk);
@@ -214,8 +219,7 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
         const int4          last = gr.back();
         std::vector<int>    un = download(c->lay.unionList.p, last.z + last.w);
         std::vector<float4> sv = download(c->shiftVec.p, kNumShifts);
-        std::vector<int>    eo = download(c->exclOff.p, na + 1);
-        std::vector<int>    ei = download(c->exclIdx.p, eo[na]);
+        std::vector<int2>   ep = download(c->exclPairSlots.p, c->numExclPairs);
 
         hXq.insert(hXq.end(), xq.begin(), xq.begin() + 4 * nc);
         hType.insert(hType.end(), ty.begin(), ty.begin() + 4 * nc);
@@ -228,10 +232,6 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
         for (int v : ai)
         {
             hAi.push_back(v >= 0 ? v + atomOffset : -1);
-        }
-        for (int v : ce)
-        {
-            hCells.push_back(v + 4 * clusterOff);
         }
         for (uint2 e : wk)
         {
@@ -255,28 +255,32 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
         }
         hShift.insert(hShift.end(), sv.begin(), sv.end());
         hChunkShift.insert(hChunkShift.end(), cs.begin(), cs.end());
-        for (int k = 0; k < na; k++)
-        {
-            hExOff.push_back(hExOff.back() + (eo[k + 1] - eo[k]));
-            hAtomSys.push_back(r);
-        }
-        for (int v : ei)
-        {
-            hExIdx.push_back(v + atomOffset);
-        }
         maxSlots = std::max(maxSlots, c->lay.windowSlots);
         anySpill = anySpill || c->lay.spill;
         ncj += c->ncj;
         clusterOff += nc;
         atomOffset += na;
         hGroupOff.push_back(static_cast<int>(hGroups.size()));
-        hAtomOff.push_back(atomOffset);
+        // the system's slots and excluded pairs in equal shares of workgroups
+        const int slot0 = 4 * (clusterOff - nc), pair0 = static_cast<int>(hExclPairs.size());
+        for (int2 v : ep)
+        {
+            hExclPairs.push_back(make_int2(v.x + slot0, v.y + slot0));
+        }
+        const int np = static_cast<int>(ep.size()), nblk = (std::max(4 * nc, np) + kExclBatchSlots - 1) / kExclBatchSlots;
+        for (int k = 0; k < nblk; k++)
+        {
+            auto at = [&](int n, int m) { return static_cast<int>(static_cast<long long>(n) * m / nblk); };
+            hExclBlocks.push_back(make_int4(slot0 + at(4 * nc, k), slot0 + at(4 * nc, k + 1), pair0 + at(np, k),
+                                            pair0 + at(np, k + 1)));
+            hExclSystem.push_back(r);
+        }
+        hExclOff.push_back(static_cast<int>(hExclBlocks.size()));
     }
 
     upload(b->xq, hXq);
     upload(b->nbtype, hType);
     upload(b->atomIndices, hAi);
-    upload(b->cells, hCells);
     upload(b->work, hWork);
     upload(b->chunks, hChunks);
     upload(b->groups, hGroups);
@@ -284,15 +288,16 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
     upload(b->unionList, hUnion);
     upload(b->shiftVec, hShift);
     upload(b->chunkShift, hChunkShift);
-    upload(b->exclOff, hExOff);
-    upload(b->exclIdx, hExIdx);
-    upload(b->atomSystem, hAtomSys);
+    upload(b->exclPairSlots, hExclPairs);
+    upload(b->exclBlockSystem, hExclSystem);
     upload(b->groupOff, hGroupOff);
-    upload(b->atomOff, hAtomOff);
+    upload(b->exclBlockOff, hExclOff);
+    upload(b->exclBlocks, hExclBlocks);
+    b->numExclBlocks = static_cast<int>(hExclBlocks.size());
+    b->exclPartial.ensure(std::max<size_t>(hExclBlocks.size(), 1));
     upload(b->boxes, b->boxHost);
     b->fnb.ensure(4 * static_cast<size_t>(totClusters) + 4);
     b->fixF.ensure(3 * (4 * static_cast<size_t>(totClusters) + 4));
-    b->atomEnergy.ensure(std::max(atomOffset, 1));
     b->energy.ensure(2 * static_cast<size_t>(R));
 
     b->totAtoms    = atomOffset;
@@ -355,29 +360,31 @@ void enqueueCompute(nbx_batch* b, const float* x, float* f, unsigned flags)
     a.fixF         = fix;
     a.energyPartial = b->energyPartial.p;
     a.fshiftPartial = nullptr;
+    if (energy)
+    {
+        // the self and excluded-pair energies, in the launch's tail
+        ExclusionArgs& e = a.excl;
+        e.xq             = b->xq.p;
+        e.pairSlots      = b->exclPairSlots.p;
+        e.elec           = c0->elec;
+        e.ic             = c0->ic;
+        e.rc2            = static_cast<double>(c0->ic.rcoulomb2);
+        e.epsfacD        = static_cast<double>(c0->ic.epsfac);
+        e.selfCoef       = c0->selfCoef;
+        e.tabD           = c0->tabFDV0d.p;
+        e.partial        = b->exclPartial.p;
+        e.blockItems     = b->exclBlocks.p;
+        e.blockSystem    = b->exclBlockSystem.p;
+        e.boxes          = b->boxes.p;
+        a.exclBlocks     = b->numExclBlocks;
+    }
     check(launchNonbonded(b->stream, a, c0->elec, energy, false, b->numBlocks), "nonbonded kernel");
     launchGatherForces(b->stream, b->totClusters, b->gather.gposOff.p, b->gather.gpos.p, b->gather.staging.p,
                        fnb, b->atomIndices.p, f, (flags & NBX_COMPUTE_ADD_FORCES) != 0, nullptr, nullptr, fix);
     if (energy)
     {
-        ExclusionArgs e{};
-        e.natoms     = b->totAtoms;
-        e.cells      = b->cells.p;
-        e.xq         = b->xq.p;
-        e.exclOff    = b->exclOff.p;
-        e.exclIdx    = b->exclIdx.p;
-        e.elec       = c0->elec;
-        e.ic         = c0->ic;
-        e.rc2        = static_cast<double>(c0->ic.rcoulomb2);
-        e.epsfacD    = static_cast<double>(c0->ic.epsfac);
-        e.selfCoef   = c0->selfCoef;
-        e.tabD       = c0->tabFDV0d.p;
-        e.atomSystem = b->atomSystem.p;
-        e.boxes      = b->boxes.p;
-        e.atomEnergy = b->atomEnergy.p;
-        launchExclusionEnergy(b->stream, e);
         launchBatchFinalize(b->stream, static_cast<int>(b->sys.size()), b->slotOff.p, b->energyPartial.p,
-                            b->atomOff.p, b->atomEnergy.p, b->energy.p);
+                            b->exclBlockOff.p, b->exclPartial.p, b->energy.p);
     }
 }
 

@@ -12,13 +12,11 @@
 //               atomdata.cpp:1471-1487) summed in double in a fixed order
 //   virial      -1/2 sum x (x) f - 1/2 sum shift (x) fshift in double
 //               (calcvir.cpp:103-148, sim_util.cpp:157-177)
-//   exclusion   the Coulomb energy terms the pair kernel leaves out, in
-//   energies    double (exclusion.h), per atom for batches; a single
-//               system's pass runs in the pair kernel's launch
+//   (the Coulomb energy terms the pair kernel leaves out run in its launch,
+//   exclusion.h)
 // All are HBM-bandwidth bound: one coalesced pass over the arrays.
 #include <algorithm>
 
-#include "exclusion.h"
 #include "kernel_common.h"
 
 namespace nbx
@@ -128,6 +126,7 @@ __global__ void reduceFKernel(int natoms, const int* __restrict__ cells, const f
 }
 
 constexpr int kFinalizeThreads = 1024;
+constexpr int kBatchFinalizeThreads = 256;
 
 // Sum of v[k * stride + comp] over k in [0, n) by this thread's share of a
 // workgroup, with four independent accumulators (the loads of one pass are
@@ -252,128 +251,45 @@ __global__ __launch_bounds__(kFinalizeThreads) void finalizeKernel(int numEnergy
     (void)doShift;
 }
 
-constexpr int kExclThreads = 256;
-
-// Atom i's self energy and the Coulomb energies of its excluded partners
-// j > i inside the cut-off, in double.
-__device__ double atomExclusionEnergy(const ExclusionArgs& a, int i)
+// Per-system energies of a batch: block r sums system r's energy slots and
+// its exclusion workgroups' sums in a fixed order.
+__global__ __launch_bounds__(kBatchFinalizeThreads) void batchFinalizeKernel(const int* __restrict__ slotOff,
+                                                                             const double* __restrict__ ePart,
+                                                                             const int* __restrict__ exclOff,
+                                                                             const double* __restrict__ exclPart,
+                                                                             double* __restrict__ eOut)
 {
-    // the atom's system box (a batch keeps one per system)
-    const float* box = a.atomSystem ? a.boxes + 3 * a.atomSystem[i] : a.box;
-    const double L[3] = { box[0], box[1], box[2] };
-    const float4 pi   = a.xq[a.cells[i]];
-    const double qi   = pi.w;
-    double       ei   = -a.selfCoef * qi * qi;
-    for (int k = a.exclOff[i]; k < a.exclOff[i + 1]; k++)
-    {
-        const int j = a.exclIdx[k];
-        if (j <= i)
-        {
-            continue;
-        }
-        const float4 pj = a.xq[a.cells[j]];
-        double       d[3] = { static_cast<double>(pi.x) - pj.x, static_cast<double>(pi.y) - pj.y,
-                        static_cast<double>(pi.z) - pj.z };
-        double       r2   = 0.0;
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-        {
-            d[c] -= L[c] * rint(d[c] / L[c]);
-            r2 += d[c] * d[c];
-        }
-        if (r2 < a.rc2)
-        {
-            const double qq = a.epsfacD * qi * static_cast<double>(pj.w);
-            if (a.elec == kElecRF)
-            {
-                ei += qq * (static_cast<double>(a.ic.k_rf) * r2 - static_cast<double>(a.ic.c_rf));
-            }
-            else
-            {
-                ei -= qq * ewaldCorrectionD(sqrt(r2), a);
-            }
-        }
-    }
-    return ei;
-}
-
-__global__ __launch_bounds__(kExclThreads) void exclusionEnergyKernel(const ExclusionArgs a)
-{
-    __shared__ double s[kExclThreads / 64];
-    double            e = 0.0;
-    for (int i = blockIdx.x * kExclThreads + threadIdx.x; i < a.natoms; i += gridDim.x * kExclThreads)
-    {
-        const double ei = atomExclusionEnergy(a, i);
-        if (a.atomEnergy)
-        {
-            a.atomEnergy[i] = ei;
-        }
-        e += ei;
-    }
-    if (a.atomEnergy)
-    {
-        return;
-    }
-#pragma unroll
-    for (int m = 1; m < 64; m *= 2)
-    {
-        e += __shfl_xor(e, m, 64);
-    }
-    if ((threadIdx.x & 63) == 0)
-    {
-        s[threadIdx.x / 64] = e;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        double t = 0.0;
-        for (int w = 0; w < kExclThreads / 64; w++)
-        {
-            t += s[w];
-        }
-        a.partial[blockIdx.x] = t;
-    }
-}
-
-// Per-system energies of a batch: block r sums system r's group energies
-// and per-atom exclusion energies in a fixed order.
-__global__ __launch_bounds__(kFinalizeThreads) void batchFinalizeKernel(const int* __restrict__ slotOff,
-                                                                        const double* __restrict__ ePart,
-                                                                        const int* __restrict__ atomOff,
-                                                                        const double* __restrict__ atomEnergy,
-                                                                        double* __restrict__ eOut)
-{
-    __shared__ double s[2][kFinalizeThreads];
-    const int r = blockIdx.x;
-    double    v = 0.0, c = 0.0;
-    for (int g = slotOff[r] + threadIdx.x; g < slotOff[r + 1]; g += kFinalizeThreads)
+    constexpr int     kWaves = kBatchFinalizeThreads / 64;
+    __shared__ double s[2][kWaves];
+    const int         r = blockIdx.x;
+    double            v = 0.0, c = 0.0;
+    for (int g = slotOff[r] + threadIdx.x; g < slotOff[r + 1]; g += kBatchFinalizeThreads)
     {
         v += ePart[2 * g];
         c += ePart[2 * g + 1];
     }
-    for (int i = atomOff[r] + threadIdx.x; i < atomOff[r + 1]; i += kFinalizeThreads)
+    for (int k = exclOff[r] + threadIdx.x; k < exclOff[r + 1]; k += kBatchFinalizeThreads)
     {
-        c += atomEnergy[i];
+        c += exclPart[k];
     }
-    s[0][threadIdx.x] = v;
-    s[1][threadIdx.x] = c;
+    v = waveSumD(v);
+    c = waveSumD(c);
+    if ((threadIdx.x & 63) == 0)
+    {
+        s[0][threadIdx.x / 64] = v;
+        s[1][threadIdx.x / 64] = c;
+    }
     __syncthreads();
-    for (int off = kFinalizeThreads / 2; off > 0; off >>= 1)
+    if (threadIdx.x < 2)
     {
-        if (threadIdx.x < off)
+        double t = 0.0;
+        for (int w = 0; w < kWaves; w++)
         {
-            s[0][threadIdx.x] += s[0][threadIdx.x + off];
-            s[1][threadIdx.x] += s[1][threadIdx.x + off];
+            t += s[threadIdx.x][w];
         }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-    {
-        eOut[2 * r]     = s[0][0];
-        eOut[2 * r + 1] = s[1][0];
+        eOut[2 * r + threadIdx.x] = t;
     }
 }
-
 
 // Forces of each cluster from the staged windows that hold it: a wavefront
 // per cluster, lane l adding copies l, l + 64, ... (12 floats each), then a
@@ -716,22 +632,14 @@ void launchExclusionSlots(hipStream_t s, int npairs, const int2* pairs, const in
 }
 
 void launchBatchFinalize(hipStream_t s, int numSystems, const int* slotOff, const double* energyPartial,
-                         const int* atomOff, const double* atomEnergy, double* energyOut)
+                         const int* exclOff, const double* exclPartial, double* energyOut)
 {
     if (numSystems > 0)
     {
-        batchFinalizeKernel<<<numSystems, kFinalizeThreads, 0, s>>>(slotOff, energyPartial, atomOff, atomEnergy,
-                                                                    energyOut);
+        batchFinalizeKernel<<<numSystems, kBatchFinalizeThreads, 0, s>>>(slotOff, energyPartial, exclOff, exclPartial,
+                                                                         energyOut);
     }
 }
-
-int launchExclusionEnergy(hipStream_t s, const ExclusionArgs& a)
-{
-    const int blocks = std::max(1, std::min(kExclMaxBlocks, (a.natoms + kExclThreads - 1) / kExclThreads));
-    exclusionEnergyKernel<<<blocks, kExclThreads, 0, s>>>(a);
-    return blocks;
-}
-
 
 void launchExpandPairs(hipStream_t s, const int4* ientry, int nci, const uint2* jentry, const float4* xq,
                        const int* atomIndices, const float4* shiftVec, float r2, unsigned long long* counter,

@@ -398,11 +398,7 @@ void launchSystemSlots(hipStream_t s, int numSystems, const int* groupOff, int n
 // the self energy and excluded-pair Coulomb energies in double
 struct ExclusionArgs
 {
-    int              natoms;
-    const int*       cells;
     const float4*    xq;
-    const int*       exclOff;
-    const int*       exclIdx;
     float            box[3];
     int              elec;
     InteractionConst ic;
@@ -411,13 +407,13 @@ struct ExclusionArgs
     double           selfCoef; // epsfac V(0) / 2
     const double*    tabD;     // FDV0 table in double (table flavour)
     double*          partial;  // one per block
-    // batches: the atom's system (boxes[3 * system]) and per-atom energies
-    // instead of block partials; nullptr for a single system
-    const int*       atomSystem;
+    // batches: per block {first slot, end, first pair, end} and its system,
+    // and the systems' boxes; nullptr for a single system
+    const int4*      blockItems;
+    const int*       blockSystem;
     const float*     boxes;
-    double*          atomEnergy;
-    // single system, pair form: nslot cluster slots (self terms) and npairs
-    // excluded pairs as cluster slots
+    // nslot cluster slots (self terms) and npairs excluded pairs as cluster
+    // slots
     int              nslot;
     int              npairs;
     const int2*      pairSlots;
@@ -464,7 +460,7 @@ struct KernelArgs
     int      waveEnergy;
     float*   fshiftPartial; // [gridDim.x - exclBlocks][45*3]
     // with energies: the last exclBlocks workgroups of the launch run the
-    // single-system exclusion pass instead (partials excl.partial[0,
+    // exclusion pass instead (partials excl.partial[0,
     // exclBlocks)), in the tail the pair workgroups leave; 0 for none
     int           exclBlocks;
     ExclusionArgs excl;
@@ -563,12 +559,14 @@ void launchFinalize(hipStream_t s, int numEnergyPartials, const double* energyPa
                     double* energyOut, double* fshiftOut, int numVirPartials, const double* virPartial,
                     const float4* shiftVec, double* virialOut);
 constexpr int kExclMaxBlocks = 1024;
-// per-atom form (batches: per-atom energies or block partials)
-int launchExclusionEnergy(hipStream_t s, const ExclusionArgs& a);
+// cluster slots per workgroup of a batch's exclusion pass
+constexpr int kExclBatchSlots = 2048;
 // the excluded pairs (atom indices, each pair once) as cluster slots
 void launchExclusionSlots(hipStream_t s, int npairs, const int2* pairs, const int* cells, int2* pairSlots);
+// per-system energies of a batch: energy slots [slotOff[r], slotOff[r + 1])
+// and exclusion partials [exclOff[r], exclOff[r + 1]) of system r
 void launchBatchFinalize(hipStream_t s, int numSystems, const int* slotOff, const double* energyPartial,
-                         const int* atomOff, const double* atomEnergy, double* energyOut);
+                         const int* exclOff, const double* exclPartial, double* energyOut);
 void launchExpandPairs(hipStream_t s, const int4* ientry, int nci, const uint2* jentry, const float4* xq,
                        const int* atomIndices, const float4* shiftVec, float r2, unsigned long long* counter,
                        long long* out, long long cap);

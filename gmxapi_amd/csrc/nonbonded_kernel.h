@@ -347,11 +347,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     extern __shared__ float4 smem4[];
     if (kEnergy && a.exclBlocks > 0 && static_cast<int>(blockIdx.x) >= static_cast<int>(gridDim.x) - a.exclBlocks)
     {
-        // the single-system exclusion pass: these workgroups are dispatched
-        // after the pair workgroups and run where those have finished
+        // the exclusion pass: these workgroups are dispatched after the pair
+        // workgroups and run where those have finished
         const int first = static_cast<int>(gridDim.x) - a.exclBlocks;
-        exclusionPairBlock(a.excl, static_cast<int>(blockIdx.x) - first, a.exclBlocks, kThreads,
-                           reinterpret_cast<double*>(smem4));
+        exclusionBlock(a.excl, static_cast<int>(blockIdx.x) - first, a.exclBlocks, kThreads,
+                       reinterpret_cast<double*>(smem4));
         return;
     }
     const int       ntype  = a.ntype;
