@@ -870,8 +870,14 @@ int nbx_set_stream(nbx_context* c, void* stream)
     {
         return fail(NBX_ERROR_INPUT, "NULL context");
     }
-    c->stream = static_cast<hipStream_t>(stream);
-    return NBX_SUCCESS;
+    return guarded([&] {
+        if (c->stream != static_cast<hipStream_t>(stream))
+        {
+            // work on the new stream reads the parameters queued on the old one
+            c->nbfpUpload.wait();
+        }
+        c->stream = static_cast<hipStream_t>(stream);
+    });
 }
 
 int nbx_set_nonbonded_parameters(nbx_context* c, int numTypes, const double* c6, const double* c12)
@@ -909,10 +915,28 @@ int nbx_set_nonbonded_parameters(nbx_context* c, int numTypes, const double* c6,
                 nb[i * t + j] = make_float2(static_cast<float>(a) * 6.0f, static_cast<float>(b) * 12.0f);
             }
         }
-        // the stream's queued kernels may still read the old table
-        check(hipStreamSynchronize(c->stream), "sync");
-        c->nbfp.ensure(nb.size());
-        check(hipMemcpy(c->nbfp.p, nb.data(), sizeof(float2) * nb.size(), hipMemcpyHostToDevice), "upload nbfp");
+        // the stream's queued kernels may still read the old table: the new one
+        // follows them (a fit sets parameters twice per step, and each wait
+        // would drain the stream), or waits for them where tables change size,
+        // LJ-PME's second table goes along, or a batch's stream reads them
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        check(hipStreamIsCapturing(c->stream, &capturing), "sync");
+        if (capturing != hipStreamCaptureStatusNone)
+        {
+            throw DeviceError("sync: parameters cannot be set while the stream is being captured");
+        }
+        const bool follows = nb.size() <= c->nbfp.cap && c->nbfp.p && c->opt.vdw_type != NBX_VDW_PME && !c->batchMember;
+        if (follows)
+        {
+            c->nbfpUpload.copy(c->stream, c->nbfp.p, nb.data(), nb.size());
+        }
+        else
+        {
+            check(hipStreamSynchronize(c->stream), "sync");
+            c->nbfpUpload.wait();
+            c->nbfp.ensure(nb.size());
+            check(hipMemcpy(c->nbfp.p, nb.data(), sizeof(float2) * nb.size(), hipMemcpyHostToDevice), "upload nbfp");
+        }
         // per type: whether it has LJ with any type (water hydrogens do not;
         // the pair kernel skips their LJ terms, which are exactly zero)
         std::vector<int> lj(t, 0);
@@ -923,8 +947,14 @@ int nbx_set_nonbonded_parameters(nbx_context* c, int numTypes, const double* c6,
                 lj[i] |= (nb[i * t + j].x != 0.0f || nb[i * t + j].y != 0.0f) ? 1 : 0;
             }
         }
-        c->typeLJ.ensure(t);
-        check(hipMemcpy(c->typeLJ.p, lj.data(), sizeof(int) * t, hipMemcpyHostToDevice), "upload LJ flags");
+        if (lj != c->typeLJHost)
+        {
+            check(hipStreamSynchronize(c->stream), "sync");
+            c->typeLJHost.clear();
+            c->typeLJ.ensure(t);
+            check(hipMemcpy(c->typeLJ.p, lj.data(), sizeof(int) * t, hipMemcpyHostToDevice), "upload LJ flags");
+            c->typeLJHost = lj;
+        }
         c->ljMask = 0;
         for (int i = 0; i < t; i++)
         {

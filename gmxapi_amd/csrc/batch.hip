@@ -491,6 +491,7 @@ int nbx_batch_add_system(nbx_batch* b, int numAtoms, const int* types, const flo
         nbx_context* c = nullptr;
         statusCheck(nbx_create(&b->opt, &c), "nbx_create");
         b->sys.push_back(c);
+        c->batchMember = true;
         statusCheck(nbx_set_stream(c, b->stream), "nbx_set_stream");
         statusCheck(nbx_set_nonbonded_parameters(c, b->ntypes, b->c6.data(), b->c12.data()),
                     "nbx_set_nonbonded_parameters");

@@ -134,6 +134,57 @@ struct PinnedBuf
     }
 };
 
+// Two pinned buffers for small uploads that follow the stream's queued work
+// instead of waiting for it; a buffer is reused once its copy is done.
+struct UploadRing
+{
+    PinnedBuf<float2> buf[2];
+    hipEvent_t        done[2]   = { nullptr, nullptr };
+    int               next      = 0;
+    bool              unordered = false; // a copy may still be queued on the stream
+    // waits until every copy is done (for another stream, or to free)
+    void wait()
+    {
+        for (hipEvent_t e : done)
+        {
+            if (e && unordered)
+            {
+                check(hipEventSynchronize(e), "hipEventSynchronize");
+            }
+        }
+        unordered = false;
+    }
+    void copy(hipStream_t s, float2* dst, const float2* src, size_t n)
+    {
+        const int k = next;
+        next ^= 1;
+        if (done[k])
+        {
+            check(hipEventSynchronize(done[k]), "hipEventSynchronize");
+        }
+        else
+        {
+            check(hipEventCreateWithFlags(&done[k], hipEventDisableTiming), "hipEventCreate");
+        }
+        buf[k].ensure(n);
+        std::copy(src, src + n, buf[k].p);
+        unordered = true;
+        check(hipMemcpyAsync(dst, buf[k].p, sizeof(float2) * n, hipMemcpyHostToDevice, s), "upload");
+        check(hipEventRecord(done[k], s), "hipEventRecord");
+    }
+    ~UploadRing()
+    {
+        for (hipEvent_t e : done)
+        {
+            if (e)
+            {
+                (void)hipEventSynchronize(e);
+                (void)hipEventDestroy(e);
+            }
+        }
+    }
+};
+
 // The pair kernel's staged j-force windows and the lists that gather them
 // (one per context, one per batch).
 struct WindowGather
@@ -289,6 +340,9 @@ struct nbx_context
     int            ntypeUser = -1;
     int            ntype     = 0; // incl. padding
     nbx::DevBuf<float2> nbfp;
+    nbx::UploadRing     nbfpUpload;
+    std::vector<int>    typeLJHost; // what typeLJ holds
+    bool                batchMember = false; // its parameters are read on the batch's stream
     nbx::DevBuf<float4> tabFDV0;
     nbx::DevBuf<double> tabFDV0d;
     nbx::DevBuf<float4> shiftVec;

@@ -120,3 +120,35 @@ def test_adjoint_at_the_limits_of_its_lds(natoms, ntypes, correction, bar):
     for got, want in ((g6, ref["grad_c6"]), (g12, ref["grad_c12"])):
         got, want = A.symmetrized(got), A.symmetrized(want)
         assert np.abs(got - want).max() <= bar * np.abs(want).max()
+
+
+@pytest.mark.parametrize("switch_streams", [False, True])
+def test_parameters_follow_queued_steps(switch_streams):
+    # new LJ parameters are uploaded behind the stream's queued steps, which
+    # keep the ones they were queued with; a step on another stream sees the
+    # last ones set
+    import torch
+
+    s = S.water_box(1001, None, seed=4)
+    m6, m12 = nbx.nblib_c6c12_matrices(s.c6, s.c12)
+    scales = [1.0, 1.5, 0.5, 1.25, 0.75, 1.1]
+    want = []
+    for k in scales:
+        ctx = nbx.context_for(s)
+        ctx.set_nonbonded_parameters(k * m6, k * m12)
+        want.append(ctx.compute(s.x))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    x = torch.from_numpy(s.x.astype(np.float32)).cuda()
+    out = [torch.empty_like(x) for _ in scales]
+    torch.cuda.synchronize()
+    ctx = nbx.context_for(s)
+    ctx.set_stream(streams[0].cuda_stream)
+    for n, k in enumerate(scales):
+        ctx.set_nonbonded_parameters(k * m6, k * m12)
+        if switch_streams:
+            ctx.synchronize()  # the steps share the context's buffers
+            ctx.set_stream(streams[n % 2].cuda_stream)
+        ctx.compute_device(x.data_ptr(), out[n].data_ptr())
+    torch.cuda.synchronize()
+    for got, w in zip(out, want):
+        assert rms(got.cpu().numpy() - w) <= 4e-6 * rms(w)
