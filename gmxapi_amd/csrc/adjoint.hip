@@ -1,7 +1,7 @@
 // Adjoint of the cluster-pair forces: the vector-Jacobian product of the
 // pair kernel's forces with a per-atom input g = dL/dF (gfx950, wave64).
 //
-// The pair kernel (kernel.hip) adds f_ij = s(r^2; q, C6, C12) d_ij to atom i
+// The pair kernel (nonbonded_kernel.h) adds f_ij = s(r^2; q, C6, C12) d_ij to atom i
 // and subtracts it from atom j, with d_ij = x_i + shift - x_j and
 //   s = 12 C12 r^-14 - 6 C6 r^-8 + epsfac q_i q_j h(r),
 // h(r) = r^-3 (non-excluded pairs only) minus the Ewald correction's force

