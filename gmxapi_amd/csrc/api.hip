@@ -1635,19 +1635,14 @@ static void enqueueStep(nbx_context* c, unsigned flags, const float* xd, float* 
     c->haveEnergy = energy;
     c->haveShift  = shift;
     c->haveVirial = virial;
-    c->resultsRead = false;
 }
 
-// The step's results in host memory: one wait for the first getter after a
-// step, none for the others.
+// The step's results in host memory.  Every getter waits: a caller's graph
+// may have replayed the step since the last one, which only the stream knows.
 static const double* stepResults(nbx_context* c)
 {
-    if (!c->resultsRead)
-    {
-        setDevice(c);
-        check(hipStreamSynchronize(c->stream), "sync");
-        c->resultsRead = true;
-    }
+    setDevice(c);
+    check(hipStreamSynchronize(c->stream), "sync");
     return c->results.p;
 }
 

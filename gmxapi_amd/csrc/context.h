@@ -414,7 +414,6 @@ struct nbx_context
     // the last step's results, written by its final sums: energies,
     // shift forces, virial
     nbx::PinnedBuf<double> results;
-    bool                   resultsRead = false; // the stream was waited for since that step
     nbx::DevBuf<double>  exclPartial;
     nbx::DevBuf<float>   fshiftPartial, fOut;
     // adjoint

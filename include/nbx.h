@@ -257,7 +257,9 @@ int nbx_compute_adjoint(nbx_context* context, const float* x, const float* g, fl
 
 /* Energies of the last compute with NBX_COMPUTE_ENERGY (gmx_enerdata_t
  * terms reduced by reduce_energies_over_lists, kernel_common.cpp:109-133):
- * LJ and Coulomb (real-space) in kJ/mol.  Synchronises. */
+ * LJ and Coulomb (real-space) in kJ/mol.  This and the two getters below wait
+ * for the context's stream in every call, so that after a replay of a step that
+ * the caller captured into a graph on that stream they give the replay's. */
 int nbx_get_energies(nbx_context* context, double* v_lj, double* v_coulomb);
 
 /* Shift forces of the last compute (nbnxn_atomdata_add_nbat_fshift_to_fshift,

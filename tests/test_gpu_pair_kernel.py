@@ -152,3 +152,52 @@ def test_parameters_follow_queued_steps(switch_streams):
     torch.cuda.synchronize()
     for got, w in zip(out, want):
         assert rms(got.cpu().numpy() - w) <= 4e-6 * rms(w)
+
+
+def _capture_step(ctx, x, f, flags):
+    """A graph of one step on a stream of its own (eager first: the launch
+    attributes and buffers are then there); returns the graph and the stream."""
+    import torch
+
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    ctx.set_stream(stream.cuda_stream)
+    ctx.compute_device(x.data_ptr(), f.data_ptr(), flags)
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        ctx.compute_device(x.data_ptr(), f.data_ptr(), flags)
+    return graph, stream
+
+
+def test_getters_wait_for_a_replayed_step():
+    # a step captured by the caller: energies, virial and shift forces are
+    # those of the last replay, also where it is still queued behind other work
+    import torch
+
+    s = S.water_box(1001, None, seed=4)
+    rng = np.random.default_rng(7)
+    moved = [(s.x + 0.01 * rng.normal(size=s.x.shape)).astype(np.float32) for _ in range(4)]
+    ctx = nbx.context_for(s)
+    want = []
+    for xm in moved:
+        f = ctx.compute(xm, energy=True, virial=True, shift_forces=True, reproducible=True)
+        want.append((f, np.array(ctx.energies()), ctx.virial(), ctx.shift_forces()))
+    flags = (nbx.COMPUTE_FORCES | nbx.COMPUTE_ENERGY | nbx.COMPUTE_SHIFT_FORCES | nbx.COMPUTE_VIRIAL
+             | nbx.COMPUTE_REPRODUCIBLE)
+    x = torch.from_numpy(s.x.astype(np.float32)).cuda()
+    xs = [torch.from_numpy(xm).cuda() for xm in moved]
+    f = torch.zeros_like(x)
+    busy = torch.ones(4096, 4096, device="cuda")
+    graph, stream = _capture_step(ctx, x, f, flags)
+    for n, (wf, we, wv, ws) in enumerate(want):
+        print(f"[replay] {n}", flush=True)
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                busy = busy @ busy * 0.0 + 1.0
+            x.copy_(xs[n])
+            graph.replay()
+            np.testing.assert_array_equal(np.array(ctx.energies()), we)
+            np.testing.assert_array_equal(ctx.virial(), wv)
+            np.testing.assert_array_equal(ctx.shift_forces(), ws)
+            np.testing.assert_array_equal(f.cpu().numpy(), wf)
