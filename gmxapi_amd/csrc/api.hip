@@ -953,12 +953,14 @@ int nbx_set_nonbonded_parameters(nbx_context* c, int numTypes, const double* c6,
             c->typeLJHost.clear();
             c->typeLJ.ensure(t);
             check(hipMemcpy(c->typeLJ.p, lj.data(), sizeof(int) * t, hipMemcpyHostToDevice), "upload LJ flags");
+            unsigned long long mask = 0;
+            for (int i = 0; i < t; i++)
+            {
+                mask |= lj[i] ? 1ull << i : 0ull;
+            }
+            c->ljMask.ensure(1);
+            check(hipMemcpy(c->ljMask.p, &mask, sizeof(mask), hipMemcpyHostToDevice), "upload LJ flags");
             c->typeLJHost = lj;
-        }
-        c->ljMask = 0;
-        for (int i = 0; i < t; i++)
-        {
-            c->ljMask |= lj[i] ? 1ull << i : 0ull;
         }
         c->anyTypeWithoutLJ = std::count(lj.begin(), lj.end() - 1, 0) > 0;
         c->c6diag.assign(t, 0.0f);
@@ -1569,7 +1571,7 @@ static void enqueueStep(nbx_context* c, unsigned flags, const float* xd, float* 
     a.xq            = c->xq.p;
     a.type          = c->nbtype.p;
     a.nbfp          = c->nbfp.p;
-    a.ljMask        = c->ljMask;
+    a.ljMask        = c->ljMask.p;
     a.skipLJ        = c->anyTypeWithoutLJ ? 1 : 0;
     a.vdwModifier   = c->opt.vdw_modifier;
     a.ljPme         = c->opt.vdw_type == NBX_VDW_PME ? 1 : 0;

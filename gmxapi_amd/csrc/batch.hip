@@ -342,7 +342,7 @@ void enqueueCompute(nbx_batch* b, const float* x, float* f, unsigned flags)
     a.xq           = b->xq.p;
     a.type         = b->nbtype.p;
     a.nbfp         = c0->nbfp.p;
-    a.ljMask       = c0->ljMask;
+    a.ljMask       = c0->ljMask.p;
     a.skipLJ       = c0->anyTypeWithoutLJ ? 1 : 0;
     a.vdwModifier  = c0->opt.vdw_modifier;
     a.ljPme        = c0->opt.vdw_type == NBX_VDW_PME ? 1 : 0;

@@ -341,7 +341,7 @@ struct nbx_context
     int            ntype     = 0; // incl. padding
     nbx::DevBuf<float2> nbfp;
     nbx::UploadRing     nbfpUpload;
-    std::vector<int>    typeLJHost; // what typeLJ holds
+    std::vector<int>    typeLJHost; // what typeLJ and ljMask hold
     bool                batchMember = false; // its parameters are read on the batch's stream
     nbx::DevBuf<float4> tabFDV0;
     nbx::DevBuf<double> tabFDV0d;
@@ -390,7 +390,7 @@ struct nbx_context
     // group size, sized for its larger window per cluster slot; built on
     // the first adjoint call after a search)
     nbx::DevBuf<int>    typeLJ; // per type (padding type included): 1 if it has LJ with any type
-    unsigned long long  ljMask = 0; // typeLJ as bits (at most kMaxTypes + 1 types)
+    nbx::DevBuf<unsigned long long> ljMask; // one: typeLJ as bits (at most kMaxTypes + 1 types)
     bool                anyTypeWithoutLJ = false; // among the user's types
     // LJ-PME: the grid's 6 C6 per type pair; the host's 6 C6 diagonal and
     // the per-type atom counts give the self energy

@@ -433,7 +433,9 @@ struct KernelArgs
     const float4* xq;
     const int*    type;
     const float2* nbfp;
-    unsigned long long ljMask; // bit t: type t has LJ with any type
+    // one: bit t: type t has LJ with any type; in device memory, so that a
+    // replayed launch sees the parameters set last, as it does in nbfp
+    const unsigned long long* ljMask;
     int           skipLJ; // host: some type has no LJ (launch the variant that skips it)
     int           vdwModifier; // host: NBX_VDW_* modifier
     int           ljPme;       // host: LJ-PME (c6grid is read)

@@ -397,6 +397,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int t = threadIdx.x + k * kThreads;
         tabReg[k]   = tableEntry(min(t, tabN - 1));
     }
+    const auto ljMask = scalarLoad<unsigned long long>(a.ljMask);
     const int chAll0 = uniformInt(ws.x);
     const int chAll1 = uniformInt(wsEnd);
     const int gFirst = uniformInt(ws.y);
@@ -542,7 +543,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 I.q[i] = p[4 * i + 3];
                 // byte offset of the type's row in the LJ table
                 I.tOff[i] = q[i] * ntype * static_cast<int>(sizeof(float2));
-                I.lj[i]   = static_cast<int>((a.ljMask >> q[i]) & 1u);
+                I.lj[i]   = static_cast<int>((ljMask >> q[i]) & 1u);
             }
             sv = make_float4(uniformFloat(s.x), uniformFloat(s.y), uniformFloat(s.z), 0.0f);
 #pragma unroll

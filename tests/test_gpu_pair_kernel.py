@@ -201,3 +201,36 @@ def test_getters_wait_for_a_replayed_step():
             np.testing.assert_array_equal(ctx.virial(), wv)
             np.testing.assert_array_equal(ctx.shift_forces(), ws)
             np.testing.assert_array_equal(f.cpu().numpy(), wf)
+
+
+@pytest.mark.parametrize("energy", [False, True])
+def test_replayed_step_takes_the_parameters_set_last(energy):
+    # a captured step reads the LJ parameters from the context's tables: set
+    # after the capture they hold for the replays, also for a type that had no
+    # LJ then (water's hydrogens) or has none any more
+    import torch
+
+    s = S.water_box(1001, None, seed=4)
+    m6, m12 = nbx.nblib_c6c12_matrices(s.c6, s.c12)
+    every = nbx.nblib_c6c12_matrices(np.maximum(s.c6, 1e-4), np.maximum(s.c12, 1e-8))
+    sets = [(m6, m12), every, (0.5 * m6, 0.5 * m12), (0.0 * m6, 0.0 * m12), (m6, m12)]
+    want = []
+    for c6, c12 in sets:
+        ctx = nbx.context_for(s)
+        ctx.set_nonbonded_parameters(c6, c12)
+        want.append((ctx.compute(s.x, energy=True), np.array(ctx.energies())))
+    assert rms(want[1][0] - want[0][0]) > 1e-2 * rms(want[0][0])  # the hydrogens' LJ shows
+    ctx = nbx.context_for(s)
+    x = torch.from_numpy(s.x.astype(np.float32)).cuda()
+    f = torch.zeros_like(x)
+    graph, stream = _capture_step(ctx, x, f, nbx.COMPUTE_FORCES | (nbx.COMPUTE_ENERGY if energy else 0))
+    for n, ((c6, c12), (wf, we)) in enumerate(zip(sets, want)):
+        print(f"[replay] parameters {n}", flush=True)
+        ctx.set_nonbonded_parameters(c6, c12)
+        with torch.cuda.stream(stream):
+            graph.replay()
+            got = f.cpu().numpy()
+        # the forces-only kernel's sums differ by rounding (above)
+        assert rms(got - wf) <= 4e-6 * rms(wf)
+        if energy:
+            np.testing.assert_allclose(ctx.energies(), we, rtol=1e-12)
