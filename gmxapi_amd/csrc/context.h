@@ -142,16 +142,27 @@ struct UploadRing
     hipEvent_t        done[2]   = { nullptr, nullptr };
     int               next      = 0;
     bool              unordered = false; // a copy may still be queued on the stream
-    // waits until every copy is done (for another stream, or to free)
+    // waits until every copy is done (for another stream, or to free); also
+    // while the thread captures another stream, where the default mode would
+    // refuse the wait and end the capture (the copies are never captured)
     void wait()
     {
+        if (!unordered)
+        {
+            return;
+        }
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        check(hipThreadExchangeStreamCaptureMode(&mode), "capture mode");
+        hipError_t failed = hipSuccess;
         for (hipEvent_t e : done)
         {
-            if (e && unordered)
+            if (e && failed == hipSuccess)
             {
-                check(hipEventSynchronize(e), "hipEventSynchronize");
+                failed = hipEventSynchronize(e);
             }
         }
+        check(hipThreadExchangeStreamCaptureMode(&mode), "capture mode");
+        check(failed, "hipEventSynchronize");
         unordered = false;
     }
     void copy(hipStream_t s, float2* dst, const float2* src, size_t n)

@@ -234,3 +234,33 @@ def test_replayed_step_takes_the_parameters_set_last(energy):
         assert rms(got - wf) <= 4e-6 * rms(wf)
         if energy:
             np.testing.assert_allclose(ctx.energies(), we, rtol=1e-12)
+
+
+def test_stream_switch_inside_a_capture_after_new_parameters():
+    # the context moves to the captured stream inside the capture, with
+    # parameters set on its last stream (their upload is waited for, not captured)
+    import torch
+
+    s = S.water_box(1001, None, seed=4)
+    m6, m12 = nbx.nblib_c6c12_matrices(s.c6, s.c12)
+    ctx = nbx.context_for(s)
+    want = []
+    for k in (1.5, 0.5):
+        ctx.set_nonbonded_parameters(k * m6, k * m12)
+        want.append(ctx.compute(s.x))
+    x = torch.from_numpy(s.x.astype(np.float32)).cuda()
+    f = torch.zeros_like(x)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    ctx.set_stream(streams[0].cuda_stream)
+    ctx.set_nonbonded_parameters(1.5 * m6, 1.5 * m12)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[1]):
+        ctx.set_stream(streams[1].cuda_stream)
+        ctx.compute_device(x.data_ptr(), f.data_ptr())
+    for n, k in enumerate((1.5, 0.5, 1.5)):
+        ctx.set_nonbonded_parameters(k * m6, k * m12)
+        with torch.cuda.stream(streams[1]):
+            graph.replay()
+            got = f.cpu().numpy()
+        assert rms(got - want[n % 2]) <= 4e-6 * rms(want[n % 2])
