@@ -302,6 +302,17 @@ const float* deviceCoordinates(nbx_context* c, const float* x, int onDevice)
     return c->x.p;
 }
 
+bool streamCapturing(const nbx_context* c)
+{
+    if (!c->stream)
+    {
+        return false; // the null stream cannot be captured
+    }
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    check(hipStreamIsCapturing(c->stream, &status), "sync");
+    return status != hipStreamCaptureStatusNone;
+}
+
 // The list build's sizing reads: kStatsHead ints of scan totals, then the
 // per-workgroup maxima of launchPartialMax, which the kernels write straight
 // to the calling thread's pinned buffer: one stream wait, no copies.
@@ -918,14 +929,14 @@ int nbx_set_nonbonded_parameters(nbx_context* c, int numTypes, const double* c6,
         // the stream's queued kernels may still read the old table: the new one
         // follows them (a fit sets parameters twice per step, and each wait
         // would drain the stream), or waits for them where tables change size,
-        // LJ-PME's second table goes along, or a batch's stream reads them
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        check(hipStreamIsCapturing(c->stream, &capturing), "sync");
-        if (capturing != hipStreamCaptureStatusNone)
+        // LJ-PME's second table goes along, or another stream may read them
+        // next: a batch's, or the one a graph is replayed on
+        if (streamCapturing(c))
         {
             throw DeviceError("sync: parameters cannot be set while the stream is being captured");
         }
-        const bool follows = nb.size() <= c->nbfp.cap && c->nbfp.p && c->opt.vdw_type != NBX_VDW_PME && !c->batchMember;
+        const bool follows = nb.size() <= c->nbfp.cap && c->nbfp.p && c->opt.vdw_type != NBX_VDW_PME && !c->batchMember
+                             && !c->captured;
         if (follows)
         {
             c->nbfpUpload.copy(c->stream, c->nbfp.p, nb.data(), nb.size());
@@ -1545,6 +1556,7 @@ static void enqueueStep(nbx_context* c, unsigned flags, const float* xd, float* 
 {
     const bool energy = (flags & NBX_COMPUTE_ENERGY) != 0;
     const bool shift  = (flags & (NBX_COMPUTE_SHIFT_FORCES | NBX_COMPUTE_VIRIAL)) != 0;
+    c->captured       = c->captured || streamCapturing(c);
     // the virial needs the atom-order forces and coordinates of this step
     const bool virial = (flags & NBX_COMPUTE_VIRIAL) != 0 && fOut && xd;
     // one energy slot per wavefront
@@ -1796,7 +1808,7 @@ int nbx_compute_adjoint(nbx_context* c, const float* x, const float* g, float* g
         {
             throw InputError("the adjoint's j-cluster window does not fit in LDS: choose a smaller kernel_group_size");
         }
-        setDevice(c);
+        c->captured        = c->captured || streamCapturing(c);
         const size_t na    = static_cast<size_t>(c->natoms);
         const int    nslot = c->ncluster * kClusterSize;
         const float* xd    = deviceCoordinates(c, x, onDevice);

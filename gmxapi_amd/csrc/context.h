@@ -354,6 +354,7 @@ struct nbx_context
     nbx::UploadRing     nbfpUpload;
     std::vector<int>    typeLJHost; // what typeLJ and ljMask hold
     bool                batchMember = false; // its parameters are read on the batch's stream
+    bool                captured    = false; // a graph holds launches that read them, on any stream
     nbx::DevBuf<float4> tabFDV0;
     nbx::DevBuf<double> tabFDV0d;
     nbx::DevBuf<float4> shiftVec;

@@ -264,3 +264,31 @@ def test_stream_switch_inside_a_capture_after_new_parameters():
             graph.replay()
             got = f.cpu().numpy()
         assert rms(got - want[n % 2]) <= 4e-6 * rms(want[n % 2])
+
+
+def test_parameters_are_in_place_for_a_replay_on_another_stream():
+    # with a step in a graph, set_nonbonded_parameters returns when the tables
+    # hold the new parameters: the graph may be replayed on any stream next,
+    # without the context's own stream having been waited for
+    import torch
+
+    s = S.water_box(1001, None, seed=4)
+    m6, m12 = nbx.nblib_c6c12_matrices(s.c6, s.c12)
+    scales = [1.5, 0.5, 1.25, 1.0]
+    ctx = nbx.context_for(s)
+    want = []
+    for k in scales:
+        ctx.set_nonbonded_parameters(k * m6, k * m12)
+        want.append(ctx.compute(s.x))
+    x = torch.from_numpy(s.x.astype(np.float32)).cuda()
+    f = torch.zeros_like(x)
+    graph, stream = _capture_step(ctx, x, f, nbx.COMPUTE_FORCES)
+    own = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    ctx.set_stream(own.cuda_stream)
+    for k, w in zip(scales, want):
+        ctx.set_nonbonded_parameters(k * m6, k * m12)
+        with torch.cuda.stream(stream):
+            graph.replay()
+            got = f.cpu().numpy()
+        assert rms(got - w) <= 4e-6 * rms(w)
