@@ -126,7 +126,8 @@ def test_adjoint_at_the_limits_of_its_lds(natoms, ntypes, correction, bar):
 def test_parameters_follow_queued_steps(switch_streams):
     # new LJ parameters are uploaded behind the stream's queued steps, which
     # keep the ones they were queued with; a step on another stream sees the
-    # last ones set
+    # last ones set, also where their upload is still behind the old stream's
+    # work when the context moves
     import torch
 
     s = S.water_box(1001, None, seed=4)
@@ -140,14 +141,19 @@ def test_parameters_follow_queued_steps(switch_streams):
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     x = torch.from_numpy(s.x.astype(np.float32)).cuda()
     out = [torch.empty_like(x) for _ in scales]
+    busy = torch.ones(4096, 4096, device="cuda")
     torch.cuda.synchronize()
     ctx = nbx.context_for(s)
     ctx.set_stream(streams[0].cuda_stream)
     for n, k in enumerate(scales):
-        ctx.set_nonbonded_parameters(k * m6, k * m12)
         if switch_streams:
             ctx.synchronize()  # the steps share the context's buffers
-            ctx.set_stream(streams[n % 2].cuda_stream)
+            with torch.cuda.stream(streams[n % 2]):
+                for _ in range(20):
+                    busy = busy @ busy * 0.0 + 1.0
+        ctx.set_nonbonded_parameters(k * m6, k * m12)
+        if switch_streams:
+            ctx.set_stream(streams[(n + 1) % 2].cuda_stream)
         ctx.compute_device(x.data_ptr(), out[n].data_ptr())
     torch.cuda.synchronize()
     for got, w in zip(out, want):
