@@ -90,9 +90,10 @@ __host__ __device__ inline int adjointAccCopies(int ntype)
     return ntype <= 24 ? NBX_ADJ_ACC_COPIES : 1;
 }
 // rsq floor for float (pairlist.h:146): r > 6.2e-4 nm; and a cap far beyond
-// any cut-off that keeps products of the masked 1/r = 0 finite
+// any cut-off (and the padding cluster's 3e12) that keeps what is multiplied
+// by the masked 1/r = 0 finite, (beta_lj^2 rsq)^2 of LJ-PME the largest
 constexpr float kMinRsq = 3.82e-07f;
-constexpr float kMaxRsq = 1e30f;
+constexpr float kMaxRsq = 1e15f;
 
 // Coulomb flavours of the kernel
 enum Elec : int

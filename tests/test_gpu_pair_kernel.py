@@ -37,13 +37,18 @@ def test_forces_only_kernel_matches_energy_kernel(name, options):
         assert rms(f - r64["f"]) <= 5e-4 * rms(r64["f"])
 
 
+@pytest.mark.parametrize("options", [dict(), dict(ewald_correction="analytical"), dict(coulomb="reaction-field"),
+                                     dict(vdw_modifier="force-switch", rvdw_switch=0.7),
+                                     dict(vdw_modifier="potential-switch", rvdw_switch=0.7), dict(vdw_type="pme"),
+                                     dict(vdw_cutoff=0.8)],
+                         ids=["table", "analytical", "rf", "force-switch", "potential-switch", "lj-pme", "twin"])
 @pytest.mark.parametrize("far", [1e6, 1e19, 3e38])
-def test_atom_far_outside_leaves_the_others_finite(far):
+def test_atom_far_outside_leaves_the_others_finite(far, options):
     # an atom that has left the box by any float distance is beyond every
     # cut-off: the atoms listed with it keep the forces they have without it
-    print(f"[far atom] {far}", flush=True)
+    print(f"[far atom] {far} {options}", flush=True)
     s = S.water_box(500, None, seed=6)
-    ctx = nbx.context_for(s)
+    ctx = nbx.context_for(s, **options)
     x = s.x.astype(np.float32)
     x[7] = (1e5, 1e5, 1e5)
     near = ctx.compute(x)
