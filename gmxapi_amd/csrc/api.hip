@@ -399,10 +399,10 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
     // (otherwise only for groups wider than its bitmap): for tests
     const char* sortEnv     = std::getenv("NBX_UNION_SORT");
     const bool  unionBySort = sortEnv != nullptr && sortEnv[0] == '1';
-    // a layout rebuilt for a new list starts from the size its last build
-    // chose: the sizes above it did not fit then and, for a system that
-    // moved by a few steps, do not fit now (saves a count pass per search)
-    const int largest = L.groupSize > 0 ? std::min(L.groupSize, stagedGroupSize(c, adjoint)) : stagedGroupSize(c, adjoint);
+    // a layout rebuilt for a new list leaves out the sizes that did not fit in
+    // an earlier build: for a system that moved by a few steps they do not fit
+    // now (saves a group pass and its wait per search)
+    const int largest = std::min(L.fitLimit, stagedGroupSize(c, adjoint));
     int       first   = 0;
     while (forced <= 0 && first < kGroupSizeCount - 1 && (kGroupSizeMax >> first) > largest)
     {
@@ -529,6 +529,10 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
             c->jentry.swap(c->jentryTmp);
         }
         buildOccurrences(c->stream, L.gather, ng, L.groups.p, L.groupInfo.p, L.unionList.p, nc, nc + unionTotal, true);
+        if (forced <= 0 && k > first)
+        {
+            L.fitLimit = G;
+        }
         L.groupSize   = G;
         L.ngroups     = ng;
         L.nchunk      = c->nci;
@@ -1083,8 +1087,8 @@ int nbx_set_topology(nbx_context* c, int numAtoms, const int* types, const float
             }
         }
         setDevice(c);
-        c->natoms        = numAtoms;
-        c->lay.groupSize = c->adj.groupSize = 0; // another system: its layouts choose anew
+        c->natoms       = numAtoms;
+        c->lay.fitLimit = c->adj.fitLimit = kGroupSizeMax; // another system: its layouts choose anew
         c->type.ensure(numAtoms);
         c->charge.ensure(numAtoms);
         c->exclOff.ensure(numAtoms + 1);

@@ -282,6 +282,7 @@ inline void buildSegments(hipStream_t s, WindowGather& w, int ngroups, const int
 struct WorkLayout
 {
     int            groupSize = 0, ngroups = 0, nchunk = 0, windowSlots = 0, nwork = 0;
+    int            fitLimit  = kGroupSizeMax; // the sizes above it did not fit in an earlier build
     int            numBlocks = 0; // workgroups of kKernelWaves wavefronts (the schedule's wavefronts / 4)
     bool           spill     = false; // some union clusters lie beyond their window (global atomics)
     DevBuf<int>    unionCount, spillCount, unionOff, spillOff, unionList;

@@ -110,8 +110,10 @@ typedef struct nbx_options
     double epsilon_rf;            /* 1 */
     int    ewald_potential_shift; /* 0: sh_ewald = 0 as nblib; 1: mdrun's shift */
     int    device;                /* HIP device ordinal */
-    int    kernel_group_size;     /* i-clusters per kernel work group: 0 = largest
-                                     that fits LDS, else 1, 2, 4, 8 or 16 (tuning) */
+    int    kernel_group_size;     /* i-clusters per kernel work group: 0 = the size that
+                                     stages least (more wavefronts than groups: a small
+                                     one) or the largest below it that fits LDS, else
+                                     1, 2, 4, 8 or 16 (tuning) */
     int    kernel_blocks_per_cu;  /* resident kernel workgroups per CU: 0 = as many
                                      as LDS allows up to 4 (tuning) */
     int    vdw_modifier;          /* NBX_VDW_*, default POTENTIAL_SHIFT (nblib) */

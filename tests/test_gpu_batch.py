@@ -169,3 +169,24 @@ def test_reproducible_flag_gives_identical_forces(replicas):
     fs = _split(runs[0][0], replicas)
     for k, (f_ref, _) in enumerate(_single_results(replicas)):
         assert rms(fs[k] - f_ref) <= 1e-6 * rms(f_ref)
+
+
+def test_group_size_follows_the_batch_not_its_history():
+    # the group size weighs a system's share of the launch's wavefronts: a
+    # member that was built alone takes the larger batch's size when others join
+    systems = [S.water_box(1001, None, seed=4 + k) for k in range(12)]
+    m6, m12 = nbx.nblib_c6c12_matrices(systems[0].c6, systems[0].c12)
+    options = dict(rlist=systems[0].rlist, rcoulomb=systems[0].rcoulomb)
+
+    def add(b, some):
+        for s in some:
+            b.add_system(s.types, s.charges, s.excl_off, s.excl_idx, s.box, s.x)
+        b.construct_pairlists()
+        return [b.system(k).work_groups()["group_size"] for k in range(len(b.natoms))]
+
+    at_once = add(nbx.Batch(m6, m12, **options), systems)
+    grown = nbx.Batch(m6, m12, **options)
+    alone = add(grown, systems[:1])
+    print(f"[group size] alone {alone}, at once {at_once}", flush=True)
+    assert alone[0] < at_once[0]
+    assert add(grown, systems[1:]) == at_once
