@@ -341,7 +341,7 @@ int stagedGroupSize(const nbx_context* c, bool adjoint)
     const double nj = static_cast<double>(c->ncj) / nc;
     // the wavefronts of the launch: two per SIMD, or this system's share of a
     // batch's launch
-    const double resident = c->numCU * 2.0 * (adjoint ? kAdjointWaves : kKernelWaves);
+    const double resident = c->numCU * (adjoint ? 2.0 * kAdjointWaves : 1.0 * kKernelBlocksPerCU * kKernelWaves);
     const double waves    = !adjoint && c->batchWaves > 0 ? c->batchWaves : std::min(resident, std::max(1.0, 1.0 * c->nci));
     double       least    = 0.0;
     int          best     = 1;
@@ -543,8 +543,8 @@ void buildWorkGroups(nbx_context* c, WorkLayout& L, bool adjoint, const int* spa
     throw InputError("the j-cluster window of one cluster does not fit in LDS: the pair-list cut-off is too long, or "
                      "there are too many atom types, for this kernel");
 }
-// The layout's grid and static schedule (the workgroups that can be
-// resident, every wavefront a contiguous run of chunks of about equal cost)
+// The layout's grid and static schedule (kKernelBlocksPerCU workgroups per CU
+// or the chosen number, every wavefront a contiguous run of chunks of about equal cost)
 // and its window staging.  The pair kernel runs kKernelWaves wavefronts per
 // workgroup, the adjoint kAdjointWaves.
 void scheduleLayout(nbx_context* c, WorkLayout& L, bool adjoint)
@@ -562,7 +562,7 @@ void scheduleLayout(nbx_context* c, WorkLayout& L, bool adjoint)
     {
         const int lds      = nonbondedLdsBytes(c->ntype, c->ic.tab_n, c->elec, L.windowSlots,
                                                c->opt.vdw_type == NBX_VDW_PME);
-        const int maxPerCU = c->opt.kernel_blocks_per_cu > 0 ? c->opt.kernel_blocks_per_cu : 4;
+        const int maxPerCU = c->opt.kernel_blocks_per_cu > 0 ? c->opt.kernel_blocks_per_cu : kKernelBlocksPerCU;
         const int perCU    = std::max(1, std::min(maxPerCU, (160 * 1024) / lds));
         numWaves = std::max(1, std::min((L.nchunk + kKernelWaves - 1) / kKernelWaves, perCU * c->numCU)) * kKernelWaves;
     }

@@ -118,14 +118,15 @@ void upload(DevBuf<T>& d, const std::vector<T>& h)
     }
 }
 
-// The kernel grid (blocksPerCU workgroups per CU, at most what LDS allows)
+// The kernel grid (blocksPerCU workgroups per CU, 0 for the default, at most
+// what LDS allows)
 // and its static schedule, with chunkWeight work entries per chunk.
 void scheduleBatch(nbx_batch* b, int blocksPerCU, int chunkWeight)
 {
     nbx_context* c0    = b->sys[0];
     const int    lds   = nonbondedLdsBytes(c0->ntype, c0->ic.tab_n, c0->elec, b->windowSlots,
                                            c0->opt.vdw_type == NBX_VDW_PME);
-    const int    maxBpc = blocksPerCU > 0 ? blocksPerCU : 4;
+    const int    maxBpc = blocksPerCU > 0 ? blocksPerCU : kKernelBlocksPerCU;
     b->blocksPerCU     = std::max(1, std::min(maxBpc, (160 * 1024) / lds));
     b->numBlocks       = std::max(1, std::min((b->nchunk + kKernelWaves - 1) / kKernelWaves, b->blocksPerCU * b->numCU));
     b->chunkWeight     = chunkWeight;
@@ -170,7 +171,7 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
     {
         throw StateError("the batch holds no systems");
     }
-    // the launch's wavefronts (two workgroups per CU) by the members' sizes
+    // the launch's wavefronts by the members' sizes
     long long batchClusters = 1;
     for (nbx_context* c : b->sys)
     {
@@ -179,7 +180,7 @@ void buildBatch(nbx_batch* b, int G, int blocksPerCU, int chunkWeight)
     for (nbx_context* c : b->sys)
     {
         c->opt.kernel_group_size = G;
-        c->batchWaves = 1 + static_cast<int>(2LL * kKernelWaves * b->numCU * c->ncluster / batchClusters);
+        c->batchWaves = 1 + static_cast<int>(1LL * kKernelBlocksPerCU * kKernelWaves * b->numCU * c->ncluster / batchClusters);
         statusCheck(nbx_construct_pairlist(c), "nbx_construct_pairlist");
     }
     check(hipSetDevice(b->device), "hipSetDevice");

@@ -75,6 +75,14 @@ constexpr int kGenerationSkewMilli = 80;
 // use a CU's whole LDS
 constexpr int kKernelWaves      = 4;
 constexpr int kKernelLdsBudget  = 80 * 1024;
+// workgroups per CU that the schedule fills unless it is told otherwise, and
+// that the group size is chosen for.  Registers leave room for four (three
+// with energies and shift forces) and small windows for the LDS of as many,
+// but each further workgroup stages windows of its own: 21,000 waters' atoms,
+// analytical, rc 0.8 nm, forces 27.4, 29.3 and 31.2 us per step with two,
+// three and four, with energies and virial 40.5, 43.9 and 50.1 us; 9,000 atoms
+// with reaction field at 1.0 nm 25.6 and 26.5 us with two and three
+constexpr int kKernelBlocksPerCU = 2;
 constexpr int kAdjointLdsBudget = 160 * 1024;
 // wavefronts per adjoint workgroup, and the LDS that its group size is chosen
 // for (two resident workgroups per CU)

@@ -342,7 +342,7 @@ struct LdsLayout
 };
 
 template<int kElec, bool kEnergy, bool kShift, int kLJ, bool kFixed>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void nonbondedKernel(const KernelArgs a)
+__global__ __launch_bounds__(kThreads) void nonbondedKernel(const KernelArgs a)
 {
     extern __shared__ float4 smem4[];
     if (kEnergy && a.exclBlocks > 0 && static_cast<int>(blockIdx.x) >= static_cast<int>(gridDim.x) - a.exclBlocks)

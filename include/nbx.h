@@ -114,8 +114,9 @@ typedef struct nbx_options
                                      stages least (more wavefronts than groups: a small
                                      one) or the largest below it that fits LDS, else
                                      1, 2, 4, 8 or 16 (tuning) */
-    int    kernel_blocks_per_cu;  /* resident kernel workgroups per CU: 0 = as many
-                                     as LDS allows up to 4 (tuning) */
+    int    kernel_blocks_per_cu;  /* kernel workgroups per CU: 0 = 2, at most what LDS
+                                     allows; registers leave room for 4 at once, with
+                                     energies and shift forces for 3 (tuning) */
     int    vdw_modifier;          /* NBX_VDW_*, default POTENTIAL_SHIFT (nblib) */
     double rvdw_switch;           /* switch radius for the switches, nm, 0 <= rvdw_switch < rcoulomb */
     int    vdw_type;              /* NBX_VDW_CUTOFF (nblib) or NBX_VDW_PME (potential shift only) */

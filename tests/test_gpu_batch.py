@@ -190,3 +190,21 @@ def test_group_size_follows_the_batch_not_its_history():
     print(f"[group size] alone {alone}, at once {at_once}", flush=True)
     assert alone[0] < at_once[0]
     assert add(grown, systems[1:]) == at_once
+
+
+@pytest.mark.parametrize("energy", [False, True])
+def test_workgroups_per_cu_default_and_chosen(energy):
+    # small windows without a table leave LDS for four workgroups per CU: the
+    # default stays at the two that the group size is chosen for, a chosen
+    # number is taken, and the forces are the same sums in another order
+    systems = [S.water_box(500, None, seed=30 + k, rc=0.8, rlist=0.8) for k in range(8)]
+    xd, fd = _device_arrays(systems)
+    got = {}
+    for chosen in (0, 1, 2, 3, 4):
+        b = nbx.batch_for(systems, coulomb="reaction-field", kernel_blocks_per_cu=chosen)
+        assert b.info()["blocks_per_cu"] == (chosen or 2)
+        b.compute_device(xd.data_ptr(), fd.data_ptr(), FLAGS if energy else nbx.COMPUTE_FORCES)
+        got[chosen] = fd.cpu().numpy().reshape(-1, 3)
+    print(f"[workgroups per CU] energy {energy}", flush=True)
+    for chosen in (1, 2, 3, 4):
+        assert rms(got[chosen] - got[0]) <= 4e-6 * rms(got[0])
