@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -98,8 +99,68 @@ struct DevBuf
     ~DevBuf() { release(); }
 };
 
+// Blocks of pinned host memory, from slabs that the process's contexts share:
+// a pinned allocation and its release of its own cost every context, and every
+// member of a batch, 0.1 to 0.6 ms.  A slab serves one device; an empty one is
+// given back unless it is the last.  Any thread may call.
+class PinnedBlocks
+{
+public:
+    static constexpr size_t kBytes = 4096; // of a block
+    static PinnedBlocks& instance()
+    {
+        // not destroyed: contexts may be closed while the process ends
+        static PinnedBlocks* blocks = new PinnedBlocks;
+        return *blocks;
+    }
+    // a block for the current device
+    void* take()
+    {
+        int device = 0;
+        check(hipGetDevice(&device), "hipGetDevice");
+        std::lock_guard<std::mutex> guard(lock_);
+        auto s = std::find_if(slabs_.begin(), slabs_.end(),
+                              [&](const Slab& slab) { return slab.device == device && ~slab.used != 0; });
+        if (s == slabs_.end())
+        {
+            void* q = nullptr;
+            check(hipHostMalloc(&q, kBytes * kBlocks, hipHostMallocDefault), "hipHostMalloc");
+            s = slabs_.insert(slabs_.end(), Slab{ static_cast<char*>(q), device, 0 });
+        }
+        const int k = __builtin_ctzll(~s->used);
+        s->used |= 1ull << k;
+        return s->base + k * kBytes;
+    }
+    // takes a block back that no queued work writes or reads any more
+    void give(void* block)
+    {
+        std::lock_guard<std::mutex> guard(lock_);
+        const auto s = std::find_if(slabs_.begin(), slabs_.end(), [&](const Slab& slab) {
+            return block >= slab.base && block < slab.base + kBytes * kBlocks;
+        });
+        s->used &= ~(1ull << ((static_cast<char*>(block) - s->base) / kBytes));
+        if (s->used == 0 && slabs_.size() > 1)
+        {
+            (void)hipHostFree(s->base);
+            slabs_.erase(s);
+        }
+    }
+
+private:
+    static constexpr int kBlocks = 64; // of a slab: the bits of used
+    struct Slab
+    {
+        char*              base;
+        int                device;
+        unsigned long long used;
+    };
+    std::mutex        lock_;
+    std::vector<Slab> slabs_;
+};
+
 // Pinned host memory that kernels write directly: a step's few results need no
-// copy behind the kernels, only the wait for the stream.
+// copy behind the kernels, only the wait for the stream.  Up to a block's size
+// it is one of PinnedBlocks.
 template<typename T>
 struct PinnedBuf
 {
@@ -114,24 +175,42 @@ struct PinnedBuf
         {
             return;
         }
-        if (p)
+        release();
+        constexpr size_t kBlock = PinnedBlocks::kBytes / sizeof(T);
+        void*            q      = nullptr;
+        if (n <= kBlock)
         {
-            check(hipHostFree(p), "hipHostFree");
-            p   = nullptr;
-            cap = 0;
+            q = PinnedBlocks::instance().take();
         }
-        void* q = nullptr;
-        check(hipHostMalloc(&q, std::max<size_t>(n, 1) * sizeof(T), hipHostMallocDefault), "hipHostMalloc");
+        else
+        {
+            check(hipHostMalloc(&q, n * sizeof(T), hipHostMallocDefault), "hipHostMalloc");
+        }
         p   = static_cast<T*>(q);
-        cap = std::max<size_t>(n, 1);
+        cap = std::max(n, kBlock);
     }
-    ~PinnedBuf()
+    void release()
     {
-        if (p)
+        if (!p)
+        {
+            return;
+        }
+        if (cap * sizeof(T) > PinnedBlocks::kBytes)
         {
             (void)hipHostFree(p);
         }
+        else if (hipDeviceSynchronize() == hipSuccess)
+        {
+            PinnedBlocks::instance().give(p);
+        }
+        else
+        {
+            (void)hipGetLastError(); // queued work may still write the block: not handed on
+        }
+        p   = nullptr;
+        cap = 0;
     }
+    ~PinnedBuf() { release(); }
 };
 
 // Two pinned buffers for small uploads that follow the stream's queued work

@@ -303,3 +303,39 @@ def test_parameters_are_in_place_for_a_replay_on_another_stream():
             graph.replay()
             got = f.cpu().numpy()
         assert rms(got - w) <= 4e-6 * rms(w)
+
+
+def test_many_contexts_keep_their_own_results():
+    # contexts share pinned memory for their results (64 blocks a slab): more
+    # of them than a slab holds, destroyed and created in between, on two threads
+    from concurrent.futures import ThreadPoolExecutor
+
+    s = S.water_box(70, 2.05, seed=3, rc=0.9, rlist=1.0)
+    m6, m12 = nbx.nblib_c6c12_matrices(s.c6, s.c12)
+
+    def open_context(k):
+        ctx = nbx.context_for(s)
+        ctx.set_nonbonded_parameters((1.0 + k) * m6, (1.0 + k) * m12)
+        ctx.compute(s.x, energy=True)
+        return k, ctx
+
+    one = nbx.context_for(s)
+    one.compute(s.x, energy=True)
+    lj, coulomb = one.energies()
+
+    def check(contexts):
+        for k, ctx in contexts:
+            # LJ is linear in the parameters (float pair terms)
+            np.testing.assert_allclose(ctx.energies(), ((1.0 + k) * lj, coulomb), rtol=1e-5)
+
+    with ThreadPoolExecutor(2) as pool:
+        contexts = list(pool.map(open_context, range(140)))
+        check(contexts)
+        for _, ctx in contexts[::2]:
+            ctx.close()
+        contexts = contexts[1::2] + list(pool.map(open_context, range(140, 170)))
+        check(contexts)
+    for _, ctx in contexts:
+        ctx.close()
+    one.compute(s.x, energy=True)
+    np.testing.assert_allclose(one.energies(), (lj, coulomb), rtol=1e-12)
