@@ -1341,10 +1341,11 @@ int nbx_construct_pairlist(nbx_context* c)
         // After a first search, the fill runs without a count pass: each
         // cluster writes into a region sized from the largest count seen
         // (with a margin) and the group pass makes it compact; a cluster that
-        // outgrows it sends the search through the counted path again.
+        // outgrows it sends the search through the counted path again, as do
+        // regions that an int does not index.
         bool done      = false;
         int  searchCap = 0;
-        if (c->searchCapJ > 0)
+        if (c->searchCapJ > 0 && searchRegionsFit(nc, c->searchCapJ))
         {
             const int cap = c->searchCapJ;
             c->searchJTmp.ensure(static_cast<size_t>(nc) * cap);

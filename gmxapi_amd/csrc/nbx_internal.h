@@ -260,6 +260,14 @@ struct SearchArgs
 };
 // shift indices at or below the central one: at most 14 i-entries per cluster
 constexpr int kMaxIEntriesPerCluster = 14;
+// whether regions of cap j-entries per cluster can be indexed with an int, as
+// the search's fill and the group pass index them
+constexpr bool searchRegionsFit(int ncluster, int cap)
+{
+    return static_cast<long long>(ncluster) * cap <= 0x7fffffffLL;
+}
+static_assert(searchRegionsFit(72640, 350) && searchRegionsFit(1, 0x7fffffff), "regions below the limit");
+static_assert(!searchRegionsFit(1 << 20, 1 << 11) && !searchRegionsFit(0x7fffffff, 2), "regions beyond an int");
 void launchSearch(hipStream_t s, const SearchArgs& a, bool fill);
 // countW of a list's clusters from its i-entries (offI: ncluster + 1)
 void launchClusterWork(hipStream_t s, int ncluster, const int* offI, const int4* ientry, int* countW);
