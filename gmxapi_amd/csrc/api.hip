@@ -320,7 +320,9 @@ constexpr int kStatsHead = 4;
 static_assert(kStatsHead + kPartialMaxBlocks * partialMaxStride(2, true) <= kPinnedInts, "stats fit the pinned buffer");
 
 // the forward kernel's schedule by the measured cost model (unless the cost
-// total could overflow an int)
+// total could overflow an int).  The adjoint's goes by work entries: with the
+// model, whose constants are the forward kernel's, it took 70.2 instead of
+// 69.8 us for the 24,000-atom chains and 114.4 instead of 113.3 us for 48,000
 bool useCostModel(const nbx_context* c, bool adjoint)
 {
     return !adjoint && scheduleCostBound(c->numWork, c->nci, kCostChunk) < INT_MAX;

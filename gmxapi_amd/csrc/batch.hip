@@ -12,8 +12,8 @@
 // runs of equal cost, so small systems do not leave the GPU idle and one
 // wavefront may pass from one system to the next.  Energies are summed per
 // system in a fixed order.
-// A step (coordinate conversion, force clearing, pair kernel, exclusion
-// energies, per-system sums, force reduction) is launch-bound for small
+// A step (set-up, pair kernel with the exclusion energies in its last
+// workgroups, force gather, per-system sums) is launch-bound for small
 // systems and can be recorded once into a HIP graph and replayed.
 #include <climits>
 #include <cstring>

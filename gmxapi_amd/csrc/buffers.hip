@@ -25,8 +25,7 @@ namespace nbx
 namespace
 {
 
-// also resets the kernel's work-group counter (a fill kernel rather than a
-// memset, so that the step can be captured in a graph)
+// (a kernel rather than a memset, so that the step can be captured in a graph)
 __global__ void clearF4Kernel(float4* __restrict__ p, int n, double* __restrict__ d, int nd)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;

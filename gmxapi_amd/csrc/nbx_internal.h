@@ -62,8 +62,9 @@ constexpr int kTileJ = 16;
 // i-data set-up and i-force reduction (64 replicas of 3,000 to 48,000 atoms:
 // 1016, 939 and 980 us per step with 8, 14 and 32)
 constexpr int kChunkWeight = 14;
-// the same for the adjoint's schedule (24,000-atom Hessian-vector product:
-// 85.2 us with 8, 86.6 with 14)
+// the same for the adjoint's schedule (adjoint call with 4, 8, 14 and 20, dL/dx
+// only: 24,000-atom chains 70.4, 69.8, 71.3 and 74.7 us, 48,000 atoms 112.3,
+// 113.3, 112.4 and 114.1 us)
 constexpr int kAdjointChunkWeight = 8;
 // chunk cost model of the static schedule (1/32 tile) and the extra share of
 // the first resident generation of workgroups (1/1000)
@@ -78,10 +79,12 @@ constexpr int kKernelLdsBudget  = 80 * 1024;
 // workgroups per CU that the schedule fills unless it is told otherwise, and
 // that the group size is chosen for.  Registers leave room for four (three
 // with energies and shift forces) and small windows for the LDS of as many,
-// but each further workgroup stages windows of its own: 21,000 waters' atoms,
+// but each further workgroup stages windows of its own: 21,000-atom water,
 // analytical, rc 0.8 nm, forces 27.4, 29.3 and 31.2 us per step with two,
 // three and four, with energies and virial 40.5, 43.9 and 50.1 us; 9,000 atoms
-// with reaction field at 1.0 nm 25.6 and 26.5 us with two and three
+// with reaction field at 1.0 nm 25.6 and 26.5 us with two and three.  (A batch
+// of 32 replicas of 1,500 atoms, reaction field: 54.8 and 52.3 us; the
+// autotuner finds that.)
 constexpr int kKernelBlocksPerCU = 2;
 constexpr int kAdjointLdsBudget = 160 * 1024;
 // wavefronts per adjoint workgroup, and the LDS that its group size is chosen

@@ -50,13 +50,13 @@
 //     forces-only kernels) are staged in LDS.  A group's first cluster, size
 //     and shift table come from its groupInfo record, so one launch can cover
 //     groups of several independent systems (the batched ensemble).
-//   * Energies: float per lane over the four pairs of a tile, then double;
-//     the sum of each (wavefront, group) goes to its own slot and the
-//     finalize kernel sums the slots in order, so energies are bitwise
-//     reproducible.  The self energy
-//     and the energies of excluded pairs inside the cut-off (large terms that
-//     nearly cancel) are left to a separate double-precision pass over the
-//     exclusion lists (buffers.hip); here excluded pairs contribute forces
+//   * Energies: float per lane over an i-entry's tiles, then double; the sum
+//     of each wavefront (for a batch of each wavefront and group) goes to its
+//     own slot and the finalize kernel sums the slots in order, so energies are
+//     bitwise reproducible.  The self energy and the energies of excluded pairs
+//     inside the cut-off (large terms that nearly cancel) are left to a
+//     double-precision pass over the excluded pairs, which the launch's last
+//     workgroups run (exclusion.h); elsewhere excluded pairs contribute forces
 //     only.
 // Pair arithmetic is FP32 on the vector ALUs; no matrix instructions are used
 // (the pair interaction is not a dense contraction).

@@ -22,8 +22,10 @@
 //
 // Work decomposition: one wavefront per i-cluster; lanes take one candidate
 // cluster each, candidates and hits are compacted in candidate order with
-// ballots, so the output is deterministic.  The same kernel runs twice: a count pass (per
-// i-cluster j and i counts, scanned on the device) and a fill pass.
+// ballots, so the output is deterministic.  A first search runs the kernel twice: a
+// count pass (per i-cluster j, i and work entry counts, scanned on the device)
+// and a fill pass.  Later ones run the fill alone, into a region per cluster
+// sized from the largest count seen.
 #include <cfloat>
 #include <cstdint>
 
