@@ -1,5 +1,5 @@
 /* CPU baseline only (compiled into liboracle_bench_f32.so, never the
- * checker): the cluster-pair kernel vectorised with AVX-512 the way the
+ * oracle): the cluster-pair kernel vectorised with AVX-512 the way the
  * reference's SIMD kernels are (kernels_simd_2xmm/kernel_inner.h,
  * kernel_outer.h): whole cluster pairs per vector register, exclusion masks
  * as vector masks, the analytical Ewald correction instead of the table

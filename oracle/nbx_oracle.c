@@ -2,7 +2,7 @@
  * CPU oracle for the NBNxM short-range nonbonded path (LJ + Ewald real space).
  *
  * TEST INFRASTRUCTURE ONLY.  This file is a plain-C restatement of the
- * reference's algorithm, used as the checker for the HIP product path.  Only
+ * reference's algorithm, what the HIP product path is tested against.  Only
  * tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it.
  * The product library never links or calls it.
  *
@@ -1920,7 +1920,7 @@ void orc_kernel(orc_sys* s, int energy)
 #ifdef ORC_OMP
 void orc_add_nbat_f_to_f(const orc_sys* s, real* fout);
 
-/* The CPU baseline only (built apart with OpenMP, never the checker): the
+/* The CPU baseline only (built apart with OpenMP, never the oracle): the
  * kernel over the list with OpenMP threads, each with its own force, shift
  * force and energy outputs (nbnxn_atomdata_output_t per thread,
  * kerneldispatch.cpp:243-356), reduced over the threads afterwards as

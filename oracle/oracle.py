@@ -4,7 +4,7 @@ The oracle is a plain-C restatement of the reference's nbnxm path (grid,
 4x4 pair search, exclusion masks, the plain-C reference kernel and the force
 reduction), built in float ("f32", the reference's mixed-precision build) and
 in double ("f64", the reference's double build).  Only tests/, the smoke
-check and bench.py's CPU-baseline leg use it, and only as the checker.
+check and bench.py's CPU-baseline leg use it, and only to test against.
 
 Each method cites the reference function it stands for; the C source cites
 file:line for every step.
@@ -29,7 +29,7 @@ def build() -> None:
 
 
 def _lib(precision: str) -> C.CDLL:
-    """f32 / f64: the checker; bench_f32: the CPU-baseline build of the float
+    """f32 / f64: the oracle; bench_f32: the CPU-baseline build of the float
     oracle (-O3, AVX2/FMA, OpenMP), which only bench.py's cpu_baseline uses."""
     if precision not in ("f32", "f64", "bench_f32"):
         raise ValueError(f"precision must be f32, f64 or bench_f32, not {precision!r}")

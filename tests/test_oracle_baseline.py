@@ -1,5 +1,5 @@
 """The CPU baseline's AVX-512 kernel (bench.py's cpu_baseline on AVX-512
-hosts; not the checker) against the FP64 oracle with the exact Ewald closed
+hosts; not the oracle) against the FP64 oracle with the exact Ewald closed
 form: it must compute the same physics to float accuracy, or the baseline
 it reports would not be a step of the same workload."""
 import numpy as np
